@@ -190,6 +190,43 @@ def test_self_loops_long_rows(gpu, restate, weights):
     np.testing.assert_array_equal(bits(got.val.cpu().numpy()), bits(want.val))
 
 
+@pytest.mark.parametrize("diag", ["none", "first", "last", "two", "inf"])
+def test_gcn_norm_sequential_degrees(gpu, restate, diag):
+    """Real-valued rows around every step of the in-order degree sums (16, 64,
+    1,024 entries; more than 1,024: a workgroup with an LDS stage), columns in
+    random order, the diagonal absent, at either end or twice, negative zeros
+    and, in one case, an infinite degree: every bit of the degree and of
+    1/sqrt(degree)."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(29)
+    lens = [0, 1, 2, 15, 16, 17, 31, 47, 63, 64, 65, 79, 127, 128, 129, 1007, 1022, 1023, 1024,
+            1025, 1026, 1055, 1056, 1088, 2047, 2048, 2049, 3071, 4096, 7001]
+    n = 8000
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        m = lens[i] if i < len(lens) else 0
+        c = (i + 1 + rng.integers(0, n - 1, size=m)) % n  # never the diagonal
+        if m and diag == "first":
+            c[0] = i
+        elif m and diag == "last":
+            c[-1] = i
+        elif m and diag == "two":
+            c[rng.integers(0, m, size=2)] = i
+        x = (rng.random(m) * 3).astype(np.float32)
+        x[rng.random(m) < 0.1] = -0.0
+        if diag == "inf" and m > 20:
+            x[m // 2] = np.inf
+        ci.append(c)
+        v.append(x)
+        rp.append(rp[-1] + m)
+    a = oracle.CSR(n, n, np.array(rp, np.int32), np.concatenate(ci).astype(np.int32),
+                   np.concatenate(v))
+    _, wdeg, wdis = restate.gcn_norm(a, with_degrees=True)
+    _, deg, dis = tg.gcn_norm(_dev(gpu, a), with_degrees=True)
+    np.testing.assert_array_equal(bits(deg.cpu().numpy()), bits(wdeg))
+    np.testing.assert_array_equal(bits(dis.cpu().numpy()), bits(wdis))
+
+
 @pytest.mark.parametrize("in_off,out_off", [(0, 1), (1, 0), (1, 1), (0, 2), (3, 0)])
 def test_self_loops_pointer_alignment(gpu, restate, in_off, out_off):
     """col_ind / val inputs and outputs starting 4-12 bytes past a 16-byte

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256) void csr_check_kernel(const int32_t* __restric
 // Self-loops and normalisation
 // ---------------------------------------------------------------------------
 constexpr int kGroup = 16;      // lanes per row in the row-wise passes
-constexpr int kLongRow = 2048;  // longer rows: one workgroup each (the *_long kernels)
+constexpr int kLongRow = 1024;  // longer rows: one workgroup each (self_loop_*_long)
 constexpr int kLongBlock = 256;
 
 // Correctly rounded (round-to-nearest) float sqrt and reciprocal for
@@ -338,6 +338,55 @@ __device__ __forceinline__ void load_vec(const T* __restrict__ p, int q, T (&out
     }
 }
 
+// Adds the 16 values held by a 16-lane group (lane t holds the t-th) to d in
+// lane order, on every lane.  A value costs a DPP move and a dependent add;
+// folded into one v_add_f32_dpp the compiler puts two wait states between
+// dependent adds, which is slower.
+__device__ __forceinline__ float add16_in_order(float d, float x) {
+    static_for<0, kGroup>([&](auto t) { d = d + group_bcast<kGroup, decltype(t)::value>(x); });
+    return d;
+}
+
+// Entry t (0 <= t < len) of row i of A + I: entry t of A's row [b, ...), + 1
+// on the diagonal (has: the row holds one), or the 1 inserted at `ins` >= 0;
+// +0 past the row's end, which changes no sum that started from +0.
+__device__ __forceinline__ float self_loop_entry(const int32_t* __restrict__ col_ind,
+                                                 const float* __restrict__ val, int b, int len,
+                                                 bool has, int ins, int32_t i, int t) {
+    if (t >= len) return 0.0f;
+    if (t == ins) return 1.0f;
+    const int q = b + t - (ins >= 0 && t > ins ? 1 : 0);
+    const float x = val[q];
+    return has && col_ind[q] == i ? x + 1.0f : x;
+}
+
+// The sequential fp32 sum of row i of A + I, in row order, by a 16-lane
+// group.  Bound by the chain of dependent adds; the next 64 entries' loads are
+// in flight behind the current 64 adds.
+__device__ __forceinline__ float ordered_row_sum(const int32_t* __restrict__ col_ind,
+                                                 const float* __restrict__ val, int b, int e,
+                                                 bool has, int ins, int32_t i, int g) {
+    constexpr int kUnroll = 4;
+    const int len = e - b + (ins >= 0 ? 1 : 0);
+    float cur[kUnroll], next[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+        cur[u] = self_loop_entry(col_ind, val, b, len, has, ins, i, u * kGroup + g);
+    float d = 0.0f;
+    for (int t0 = 0; t0 < len; t0 += kUnroll * kGroup) {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+            next[u] = self_loop_entry(col_ind, val, b, len, has, ins, i,
+                                      t0 + (kUnroll + u) * kGroup + g);
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+            if (t0 + u * kGroup < len) d = add16_in_order(d, cur[u]);
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) cur[u] = next[u];
+    }
+    return d;
+}
+
 // Per row of A (n x n): has_diag, first position (row order) of a column > i,
 // the row length of A + I, and -- for gcn_norm -- the degree (sequential fp32
 // sum of A + I's row values, in row order) and 1/sqrt(deg).
@@ -349,15 +398,14 @@ __device__ __forceinline__ void load_vec(const T* __restrict__ p, int q, T (&out
 // parallel (in int64).  Other rows take the sequential path in row order.
 // Each lane of the 16-lane group reads VEC consecutive entries per step.
 template <bool NORM, int VEC>
-__global__ __launch_bounds__(256) void self_loop_info_kernel(
+__device__ __forceinline__ void self_loop_info_row(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
-    const float* __restrict__ val, int64_t n, int32_t* __restrict__ first_ins,
+    const float* __restrict__ val, int64_t row, int64_t n, int32_t* __restrict__ first_ins,
     int32_t* __restrict__ new_len, float* __restrict__ deg_out, float* __restrict__ dis_out) {
-    const int64_t row = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kGroup;
     const int g = threadIdx.x % kGroup;
     if (row >= n) return;
     const int b = row_ptr[row], e = row_ptr[row + 1];
-    if (e - b > kLongRow) return;  // self_loop_info_long_kernel
+    if (e - b > kLongRow) return;  // self_loop_info_long
     const int32_t i = static_cast<int32_t>(row);
     int has = 0;
     int first_gt = e - b;  // row-relative position of the first column > i
@@ -405,22 +453,7 @@ __global__ __launch_bounds__(256) void self_loop_info_kernel(
         if (integral && iabs + (has ? 0 : 1) <= (1ll << 24)) {
             d = static_cast<float>(isum + (has ? 0 : 1));
         } else {
-            // Sequential sum in row order of A + I: chunks of kGroup values
-            // are loaded by the group and added one by one.
-            for (int base = b; base < e; base += kGroup) {
-                const int nz = base + g;
-                float v = 0.0f;
-                if (nz < e) {
-                    v = val[nz];
-                    if (col_ind[nz] == i) v = v + 1.0f;
-                }
-                const int cnt = min(kGroup, e - base);
-                for (int t = 0; t < cnt; ++t) {
-                    if (!has && base - b + t == first_gt) d = d + 1.0f;
-                    d = d + __shfl(v, t, kGroup);
-                }
-            }
-            if (!has && first_gt == e - b) d = d + 1.0f;
+            d = ordered_row_sum(col_ind, val, b, e, has != 0, has ? -1 : first_gt, i, g);
         }
         if (g == 0) {
             const float dis = d > 0.0f ? cr_rcp(cr_sqrt(d)) : 0.0f;
@@ -595,16 +628,15 @@ __device__ __forceinline__ void copy_row_granules(const int32_t* __restrict__ co
 // (copy_row_granules; col_out and val_out 16-byte aligned); VEC = 1: one
 // entry per lane and step.
 template <bool NORM, int VEC>
-__global__ __launch_bounds__(256) void self_loop_copy_kernel(
+__device__ __forceinline__ void self_loop_copy_row(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
-    const float* __restrict__ val, int64_t n, const int32_t* __restrict__ first_ins,
+    const float* __restrict__ val, int64_t row, int64_t n, const int32_t* __restrict__ first_ins,
     const int32_t* __restrict__ row_ptr_out, const float* __restrict__ dis,
     int32_t* __restrict__ col_out, float* __restrict__ val_out) {
-    const int64_t row = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kGroup;
     const int g = threadIdx.x % kGroup;
     if (row >= n) return;
     const int b = row_ptr[row], e = row_ptr[row + 1];
-    if (e - b > kLongRow) return;  // self_loop_copy_long_kernel
+    if (e - b > kLongRow) return;  // self_loop_copy_long
     const int32_t i = static_cast<int32_t>(row);
     const int ins = first_ins[row];
     const int ob = row_ptr_out[row];
@@ -666,21 +698,21 @@ __device__ __forceinline__ T block_reduce(T v, T* lds, int op) {  // op: 0 sum, 
     return v;
 }
 
-// self_loop_info for the listed long rows: one workgroup per row (grid-stride
-// over the list).  The sequential degree (rows that fail the integral test)
-// stages 1,024 values of A + I in LDS per step and adds them in row order on
-// one thread.
+// self_loop_info for the listed long rows: one workgroup per row (workgroups
+// 0..long_blocks-1, striding over the list).  The sequential degree (rows that fail the integral test)
+// is added in row order by the first wavefront, from LDS.
 template <bool NORM, int VEC>
-__global__ __launch_bounds__(kLongBlock) void self_loop_info_long_kernel(
+__device__ __forceinline__ void self_loop_info_long(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
     const float* __restrict__ val, const int32_t* __restrict__ list,
-    const int32_t* __restrict__ count, int32_t* __restrict__ first_ins,
+    const int32_t* __restrict__ count, int long_blocks, int32_t* __restrict__ first_ins,
     int32_t* __restrict__ new_len, float* __restrict__ deg_out, float* __restrict__ dis_out) {
     __shared__ long long red64[kLongBlock / kWave];
     __shared__ int red32[kLongBlock / kWave];
-    __shared__ float stage[kLongBlock * 4];
+    constexpr int kStageVec = 4, kStage = kLongBlock * kStageVec;
+    __shared__ alignas(16) float stage[2][kStage];
     const int n_long = *count;
-    for (int li = blockIdx.x; li < n_long; li += gridDim.x) {
+    for (int li = blockIdx.x; li < n_long; li += long_blocks) {
         const int32_t i = list[li];
         const int b = row_ptr[i], e = row_ptr[i + 1];
         int has = 0, first_gt = e - b, integral = 1;
@@ -722,23 +754,53 @@ __global__ __launch_bounds__(kLongBlock) void self_loop_info_long_kernel(
             if (integral && iabs + (has ? 0 : 1) <= (1ll << 24)) {
                 d = static_cast<float>(isum + (has ? 0 : 1));
             } else {
-                for (int base = b; base < e; base += kLongBlock * 4) {
-                    const int cnt = min(kLongBlock * 4, e - base);
+                // 1,024 entries of A + I's row at a time in LDS, the next ones
+                // loaded behind the first wavefront's adds (32 entries by 8
+                // broadcast 128-bit reads): the chain of dependent adds, 4
+                // cycles each, is what a 20,000-entry row takes
+                const int ins = has ? -1 : first_gt;
+                const int len = e - b + (has ? 0 : 1);
+                float x[kStageVec];
+#pragma unroll
+                for (int u = 0; u < kStageVec; ++u)
+                    x[u] = self_loop_entry(col_ind, val, b, len, has != 0, ins, i,
+                                           u * kLongBlock + static_cast<int>(threadIdx.x));
+                for (int t0 = 0, buf = 0; t0 < len; t0 += kStage, buf ^= 1) {
+#pragma unroll
+                    for (int u = 0; u < kStageVec; ++u)
+                        stage[buf][u * kLongBlock + threadIdx.x] = x[u];
                     __syncthreads();
-                    for (int t = threadIdx.x; t < cnt; t += kLongBlock) {
-                        float x = val[base + t];
-                        if (col_ind[base + t] == i) x = x + 1.0f;
-                        stage[t] = x;
-                    }
-                    __syncthreads();
-                    if (threadIdx.x == 0) {
-                        for (int t = 0; t < cnt; ++t) {
-                            if (!has && base - b + t == first_gt) d = d + 1.0f;
-                            d = d + stage[t];
+#pragma unroll
+                    for (int u = 0; u < kStageVec; ++u)
+                        x[u] = self_loop_entry(
+                            col_ind, val, b, len, has != 0, ins, i,
+                            t0 + kStage + u * kLongBlock + static_cast<int>(threadIdx.x));
+                    if (threadIdx.x < kWave) {
+                        const int cnt = min(kStage, len - t0);
+                        f32x4 y[8], z[8];
+                        const auto load32 = [&](f32x4(&v)[8], int t) {
+#pragma unroll
+                            for (int k = 0; k < 8; ++k)
+                                v[k] = *reinterpret_cast<const f32x4*>(&stage[buf][t + 4 * k]);
+                        };
+                        const auto add32 = [&](const f32x4(&v)[8]) {
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) {
+                                d = d + v[k][0];
+                                d = d + v[k][1];
+                                d = d + v[k][2];
+                                d = d + v[k][3];
+                            }
+                        };
+                        load32(y, 0);
+                        for (int t = 0; t < cnt; t += 64) {  // (kStage % 64 == 0)
+                            load32(z, t + 32);
+                            add32(y);
+                            load32(y, min(t + 64, kStage - 32));
+                            add32(z);
                         }
                     }
                 }
-                if (!has && first_gt == e - b) d = d + 1.0f;
             }
             if (threadIdx.x == 0) {
                 deg_out[i] = d;
@@ -751,14 +813,14 @@ __global__ __launch_bounds__(kLongBlock) void self_loop_info_long_kernel(
 
 // self_loop_copy for the listed long rows: one workgroup per row.
 template <bool NORM, int VEC>
-__global__ __launch_bounds__(kLongBlock) void self_loop_copy_long_kernel(
+__device__ __forceinline__ void self_loop_copy_long(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
     const float* __restrict__ val, const int32_t* __restrict__ list,
-    const int32_t* __restrict__ count, const int32_t* __restrict__ first_ins,
+    const int32_t* __restrict__ count, int long_blocks, const int32_t* __restrict__ first_ins,
     const int32_t* __restrict__ row_ptr_out, const float* __restrict__ dis,
     int32_t* __restrict__ col_out, float* __restrict__ val_out) {
     const int n_long = *count;
-    for (int li = blockIdx.x; li < n_long; li += gridDim.x) {
+    for (int li = blockIdx.x; li < n_long; li += long_blocks) {
         const int32_t i = list[li];
         const int b = row_ptr[i], e = row_ptr[i + 1];
         const int ins = first_ins[i];
@@ -779,6 +841,48 @@ __global__ __launch_bounds__(kLongBlock) void self_loop_copy_long_kernel(
             }
         }
     }
+}
+
+// One launch for both: the first long_blocks workgroups take the listed long
+// rows, so that their serial chains run beside the other rows (16 lanes each).
+// Bound by the longest row's chain of dependent adds (about 4.7 ns each): 200,000
+// rows, 10M weighted entries, longest row 20,000: 97 us.  Before, one thread
+// per long row adding from LDS one read at a time (969 us) and a shuffle per
+// add in the other rows (195 us), in launches one after the other.  With
+// kLongRow 2,048 and two launches 99 + 86 us.
+template <bool NORM, int VEC>
+__global__ __launch_bounds__(kLongBlock) void self_loop_info_kernel(
+    const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
+    const float* __restrict__ val, int64_t n, const int32_t* __restrict__ list,
+    const int32_t* __restrict__ count, int long_blocks, int32_t* __restrict__ first_ins,
+    int32_t* __restrict__ new_len, float* __restrict__ deg_out, float* __restrict__ dis_out) {
+    if (static_cast<int>(blockIdx.x) < long_blocks) {
+        self_loop_info_long<NORM, VEC>(row_ptr, col_ind, val, list, count, long_blocks, first_ins,
+                                       new_len, deg_out, dis_out);
+        return;
+    }
+    const int64_t row = (static_cast<int64_t>(blockIdx.x - long_blocks) * kLongBlock +
+                         threadIdx.x) / kGroup;
+    self_loop_info_row<NORM, VEC>(row_ptr, col_ind, val, row, n, first_ins, new_len, deg_out,
+                                  dis_out);
+}
+
+template <bool NORM, int VEC>
+__global__ __launch_bounds__(kLongBlock) void self_loop_copy_kernel(
+    const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_ind,
+    const float* __restrict__ val, int64_t n, const int32_t* __restrict__ list,
+    const int32_t* __restrict__ count, int long_blocks, const int32_t* __restrict__ first_ins,
+    const int32_t* __restrict__ row_ptr_out, const float* __restrict__ dis,
+    int32_t* __restrict__ col_out, float* __restrict__ val_out) {
+    if (static_cast<int>(blockIdx.x) < long_blocks) {
+        self_loop_copy_long<NORM, VEC>(row_ptr, col_ind, val, list, count, long_blocks, first_ins,
+                                       row_ptr_out, dis, col_out, val_out);
+        return;
+    }
+    const int64_t row = (static_cast<int64_t>(blockIdx.x - long_blocks) * kLongBlock +
+                         threadIdx.x) / kGroup;
+    self_loop_copy_row<NORM, VEC>(row_ptr, col_ind, val, row, n, first_ins, row_ptr_out, dis,
+                                  col_out, val_out);
 }
 
 unsigned grid_for(int64_t n, int per_block = 256, int64_t cap = 1 << 20) {
@@ -945,77 +1049,34 @@ void self_loops_impl(bool norm, int64_t n, int64_t nnz, const int32_t* row_ptr,
     int32_t* long_count = long_list + n;
     if (deg_out) deg = deg_out;
     if (dis_out) dis = dis_out;
-    const unsigned blocks = static_cast<unsigned>(ceil_div(n * kGroup, 256));
-    fill_i32(long_count, 1, 0, s);
-    long_rows_kernel<<<grid_for(n), 256, 0, s>>>(row_ptr, n, long_list, long_count);
-    TG_LAUNCH_CHECK();
-    const unsigned long_grid = 8192;  // grid-stride over the (device-side) long-row list
+    // workgroups for the long rows (there are at most nnz / kLongRow), then
+    // 16 rows per workgroup for the others
+    const int long_blocks = static_cast<int>(std::min<int64_t>(nnz / kLongRow, 2048));
+    const unsigned blocks = static_cast<unsigned>(long_blocks + ceil_div(n * kGroup, kLongBlock));
+    if (long_blocks > 0) {
+        fill_i32(long_count, 1, 0, s);
+        long_rows_kernel<<<grid_for(n), 256, 0, s>>>(row_ptr, n, long_list, long_count);
+        TG_LAUNCH_CHECK();
+    }
     // 128-bit reads when both arrays are 16-byte aligned
     const bool v4 = (reinterpret_cast<uintptr_t>(col_ind) | reinterpret_cast<uintptr_t>(val)) % 16 == 0;
-    if (norm && v4)
-        self_loop_info_kernel<true, 4><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n, first_ins,
-                                                              new_len, deg, dis);
-    else if (norm)
-        self_loop_info_kernel<true, 1><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n, first_ins,
-                                                              new_len, deg, dis);
-    else if (v4)
-        self_loop_info_kernel<false, 4><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n,
-                                                               first_ins, new_len, nullptr,
-                                                               nullptr);
-    else
-        self_loop_info_kernel<false, 1><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n,
-                                                               first_ins, new_len, nullptr,
-                                                               nullptr);
-    TG_LAUNCH_CHECK();
-    if (norm && v4)
-        self_loop_info_long_kernel<true, 4><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, new_len, deg, dis);
-    else if (norm)
-        self_loop_info_long_kernel<true, 1><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, new_len, deg, dis);
-    else if (v4)
-        self_loop_info_long_kernel<false, 4><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, new_len, nullptr, nullptr);
-    else
-        self_loop_info_long_kernel<false, 1><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, new_len, nullptr, nullptr);
+    const auto info = norm ? (v4 ? self_loop_info_kernel<true, 4> : self_loop_info_kernel<true, 1>)
+                           : (v4 ? self_loop_info_kernel<false, 4>
+                                 : self_loop_info_kernel<false, 1>);
+    info<<<blocks, kLongBlock, 0, s>>>(row_ptr, col_ind, val, n, long_list, long_count,
+                                       long_blocks, first_ins, new_len, deg, dis);
     TG_LAUNCH_CHECK();
     exclusive_scan_i32(new_len, row_ptr_out, n, scan, s);
     // the copy writes 128-bit granules when both outputs are 16-byte aligned
     const bool o4 = (reinterpret_cast<uintptr_t>(col_out) | reinterpret_cast<uintptr_t>(val_out)) % 16 == 0;
     // the structure alone needs no scaling: copied as add_self_loops' structure
-    const bool scale = norm && values;
-    if (scale && o4)
-        self_loop_copy_kernel<true, 4><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n, first_ins,
-                                                              row_ptr_out, dis, col_out, val_out);
-    else if (scale)
-        self_loop_copy_kernel<true, 1><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n, first_ins,
-                                                              row_ptr_out, dis, col_out, val_out);
-    else if (o4)
-        self_loop_copy_kernel<false, 4><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n,
-                                                               first_ins, row_ptr_out, nullptr,
-                                                               col_out, val_out);
-    else
-        self_loop_copy_kernel<false, 1><<<blocks, 256, 0, s>>>(row_ptr, col_ind, val, n,
-                                                               first_ins, row_ptr_out, nullptr,
-                                                               col_out, val_out);
-    TG_LAUNCH_CHECK();
-    if (scale && o4)
-        self_loop_copy_long_kernel<true, 4><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, row_ptr_out, dis, col_out,
-            val_out);
-    else if (scale)
-        self_loop_copy_long_kernel<true, 1><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, row_ptr_out, dis, col_out,
-            val_out);
-    else if (o4)
-        self_loop_copy_long_kernel<false, 4><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, row_ptr_out, nullptr,
-            col_out, val_out);
-    else
-        self_loop_copy_long_kernel<false, 1><<<long_grid, kLongBlock, 0, s>>>(
-            row_ptr, col_ind, val, long_list, long_count, first_ins, row_ptr_out, nullptr,
-            col_out, val_out);
+    const auto copy = norm && values
+                          ? (o4 ? self_loop_copy_kernel<true, 4> : self_loop_copy_kernel<true, 1>)
+                          : (o4 ? self_loop_copy_kernel<false, 4>
+                                : self_loop_copy_kernel<false, 1>);
+    copy<<<blocks, kLongBlock, 0, s>>>(row_ptr, col_ind, val, n, long_list, long_count,
+                                       long_blocks, first_ins, row_ptr_out, dis, col_out,
+                                       val_out);
     TG_LAUNCH_CHECK();
     if (own.get()) TG_HIP(hipStreamSynchronize(s));  // own workspace is freed on return
 }
