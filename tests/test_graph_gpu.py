@@ -48,6 +48,37 @@ def test_edge_list_to_csr_bitexact(gpu, restate, n, e, dmax, seed):
     np.testing.assert_array_equal(bits(v), bits(want.val))
 
 
+@pytest.mark.parametrize("n,e,kind", [
+    (1, 1, "uniform"), (2, 5000, "uniform"), (7, 16384, "uniform"), (7, 16385, "sorted"),
+    (4096, 40000, "uniform"), (4097, 1, "uniform"), (70001, 300000, "one_row"),
+    (70001, 300000, "sorted"), (1 << 22, 50000, "uniform"), ((1 << 22) + 1, 50000, "uniform"),
+    (3, 32768, "one_row"), (3, 32769, "one_row"),   # LDS sort, the sort through memory
+    (3, 262144, "one_row"), (3, 262145, "one_row"),  # that one, the general build
+    (300000, 5000000, "hubs"),
+])
+def test_edge_list_to_csr_partition_edges(gpu, restate, n, e, kind):
+    """The partition-and-sort build at the edges of its buckets, tiles, sort
+    paths and sizes, and the general build just past them."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(n + e)
+    src = rng.integers(0, n, size=e).astype(np.int32)
+    if kind == "sorted":
+        src.sort()
+    elif kind == "one_row":
+        src[:] = n - 1
+    elif kind == "hubs":
+        src[: e // 4] = rng.integers(1000, 1020, size=e // 4)
+        src[e // 4: e // 2] = n - 1 - src[e // 4: e // 2] % 4
+        rng.shuffle(src)
+    dst = rng.integers(0, n, size=e).astype(np.int32)
+    dst[:: 7] = n - 1
+    want = restate.edge_list_to_csr(src, dst, n)
+    rp, ci, v = tg.edge_list_to_csr(*_edges(gpu, src, dst), n).to_numpy()
+    np.testing.assert_array_equal(rp, want.row_ptr)
+    np.testing.assert_array_equal(ci, want.col_ind)
+    np.testing.assert_array_equal(bits(v), bits(want.val))
+
+
 def test_edge_list_to_csr_duplicates_and_self_edges(gpu, restate):
     import tinygnn_amd as tg
     rng = np.random.default_rng(9)

@@ -14,6 +14,8 @@
 //     row of A+I, dis = 1/sqrt(deg) (correctly rounded), v' = (v*dis_i)*dis_j.
 #include "common.hpp"
 #include "device_utils.hpp"
+#include "edge_sort.hpp"
+#include "layers.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -1111,13 +1113,36 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
     require(row_ptr != nullptr, W + ": row_ptr is null");
     require(n_edges == 0 || (src && dst && col_ind && val),
             W + ": null pointer");
-    Carver probe(nullptr, 0);
-    carve_csr_ws(probe, n_nodes);
     DeviceBuffer own;
     if (workspace == nullptr) {
-        own.resize(probe.bytes());
+        own.resize(edge_list_to_csr_ws(n_nodes, n_edges));
         workspace = own.get();
         ws_bytes = own.size();
+    }
+    const auto invalid_endpoint = [&](unsigned long long bad) {
+        const int64_t e = static_cast<int64_t>(bad / 2);
+        const bool is_dst = (bad & 1) != 0;
+        int32_t v = 0;
+        TG_HIP(hipMemcpy(&v, (is_dst ? dst : src) + e, sizeof(v), hipMemcpyDeviceToHost));
+        throw std::invalid_argument(W + ": edge[" + std::to_string(e) +
+                                    "]." + (is_dst ? "dst" : "src") + " = " +
+                                    std::to_string(v) + " out of range [0, " +
+                                    std::to_string(n_nodes) + ")");
+    };
+    // Partition and sort (edge_sort.hip) where an edge fits a 32-bit key (up to
+    // 2^22 nodes), the workspace has its counters, the destinations are in
+    // range and no bucket of rows is so long that one workgroup would be the
+    // slower sort; the general build below otherwise.
+    if (edge_sort_fits(n_nodes, n_edges) && ws_bytes >= edge_sort_ws(n_nodes, n_edges)) {
+        const EdgeSortStatus h = edge_sort_count(n_nodes, n_edges, src, dst, check_dst, workspace,
+                                                 ws_bytes, s);
+        if (h.bad != ~0ull) invalid_endpoint(h.bad);
+        if (edge_sort_ready(h)) {
+            edge_sort_finish(h, n_nodes, n_edges, src, dst, row_ptr, col_ind, val, workspace,
+                             ws_bytes, s);
+            if (own.get()) TG_HIP(hipStreamSynchronize(s));
+            return;
+        }
     }
     Carver c(workspace, ws_bytes);
     CsrWs w = carve_csr_ws(c, n_nodes);
@@ -1136,16 +1161,7 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
     TG_HIP(hipMemcpyAsync(&bad, w.bad, sizeof(bad), hipMemcpyDeviceToHost, s));
     TG_HIP(hipMemcpyAsync(counts, w.counts, sizeof(counts), hipMemcpyDeviceToHost, s));
     TG_HIP(hipStreamSynchronize(s));
-    if (bad != ~0ull) {
-        const int64_t e = static_cast<int64_t>(bad / 2);
-        const bool is_dst = (bad & 1) != 0;
-        int32_t v = 0;
-        TG_HIP(hipMemcpy(&v, (is_dst ? dst : src) + e, sizeof(v), hipMemcpyDeviceToHost));
-        throw std::invalid_argument(W + ": edge[" + std::to_string(e) +
-                                    "]." + (is_dst ? "dst" : "src") + " = " +
-                                    std::to_string(v) + " out of range [0, " +
-                                    std::to_string(n_nodes) + ")");
-    }
+    if (bad != ~0ull) invalid_endpoint(bad);
     exclusive_scan_i32(w.deg, row_ptr, n_nodes, w.scan, s);
     if (n_edges > 0) {
         fill_i32(w.deg, n_nodes, 0, s);  // reused as the per-row cursor
@@ -1157,10 +1173,10 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
     if (own.get()) TG_HIP(hipStreamSynchronize(s));
 }
 
-size_t edge_list_to_csr_ws(int64_t n_nodes) {
+size_t edge_list_to_csr_ws(int64_t n_nodes, int64_t n_edges) {
     Carver c(nullptr, 0);
     carve_csr_ws(c, n_nodes);
-    return c.bytes();
+    return std::max(c.bytes(), edge_sort_ws(n_nodes, n_edges));
 }
 
 void csr_validate(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t* row_ptr,
@@ -1231,8 +1247,7 @@ void unit_self_loop_dis(int64_t n, const int32_t* row_ptr, float* dis, int32_t* 
 extern "C" {
 
 size_t tg_edge_list_to_csr_workspace_size(int64_t n_nodes, int64_t n_edges) {
-    (void)n_edges;
-    return n_nodes > 0 ? tg::edge_list_to_csr_ws(n_nodes) : 0;
+    return n_nodes > 0 ? tg::edge_list_to_csr_ws(n_nodes, n_edges) : 0;
 }
 
 int tg_edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, const int32_t* dst,

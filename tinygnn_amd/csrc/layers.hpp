@@ -21,7 +21,7 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
                       int32_t* row_ptr, int32_t* col_ind, float* val, void* workspace,
                       size_t ws_bytes, hipStream_t s, bool check_dst = true,
                       const char* who = nullptr);
-size_t edge_list_to_csr_ws(int64_t n_nodes);
+size_t edge_list_to_csr_ws(int64_t n_nodes, int64_t n_edges);
 void csr_validate(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t* row_ptr,
                   const int32_t* col_ind, hipStream_t s);
 // values = false: the structure of A + I alone (row_ptr_out, col_out; val_out
