@@ -345,3 +345,37 @@ def test_square_required(gpu):
                    np.ones(2, np.float32))
     with pytest.raises(tg.InvalidArgument, match="square"):
         tg.add_self_loops(_dev(gpu, a))
+
+
+def test_temporaries_on_streams_and_threads(gpu, restate):
+    """Calls that bring no workspace, from three threads on streams of their
+    own, again and again: their temporaries, reused in stream order, do not mix."""
+    import threading
+    import tinygnn_amd as tg
+    torch = gpu
+    want, dev = [], []
+    for seed in (31, 32, 33):
+        a = random_csr(np.random.default_rng(seed), 3000 + seed, 3000 + seed, avg_deg=8,
+                       max_deg=2500)
+        a.val[:] = np.abs(a.val) + 0.01
+        want.append(restate.gcn_norm(a))
+        dev.append(_dev(gpu, a))
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(10):
+                rp, ci, v = tg.gcn_norm(dev[k]).to_numpy()
+                if not (np.array_equal(rp, want[k].row_ptr) and
+                        np.array_equal(ci, want[k].col_ind) and
+                        np.array_equal(bits(v), bits(want[k].val))):
+                    bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

@@ -2,6 +2,7 @@
 #include "common.hpp"
 #include "device_utils.hpp"
 
+#include <mutex>
 #include <string>
 
 namespace tg {
@@ -38,6 +39,85 @@ void DeviceBuffer::reset() {
     if (p_) (void)hipFree(p_);
     p_ = nullptr;
     n_ = 0;
+}
+
+namespace {
+
+constexpr uint64_t kPoolKeep = uint64_t(512) << 20;
+
+// The current device's pool, or null where it cannot be made.
+hipMemPool_t device_pool() {
+    constexpr int kMaxDevices = 64;
+    static std::mutex mu;
+    static hipMemPool_t pools[kMaxDevices] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lock(mu);
+    if (pools[dev] == nullptr) {
+        hipMemPoolProps props{};
+        props.allocType = hipMemAllocationTypePinned;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = dev;
+        hipMemPool_t pool = nullptr;
+        if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
+        uint64_t keep = kPoolKeep;
+        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+            (void)hipMemPoolDestroy(pool);
+            return nullptr;
+        }
+        pools[dev] = pool;
+    }
+    return pools[dev];
+}
+
+}  // namespace
+
+void TempBuffer::allocate(size_t bytes, hipStream_t s) {
+    reset();
+    if (bytes == 0) return;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipMemPool_t pool = nullptr;
+    if (hipStreamIsCapturing(s, &capture) == hipSuccess &&
+        capture == hipStreamCaptureStatusNone)
+        pool = device_pool();
+    if (pool != nullptr) {
+        hipError_t e = hipMallocFromPoolAsync(&p_, bytes, pool, s);
+        if (e != hipSuccess) {  // give the pool's free memory back, then once more
+            (void)hipGetLastError();
+            (void)hipStreamSynchronize(s);
+            (void)hipMemPoolTrimTo(pool, 0);
+            e = hipMallocFromPoolAsync(&p_, bytes, pool, s);
+        }
+        if (e == hipSuccess) {
+            n_ = bytes;
+            stream_ = s;
+            pooled_ = true;
+            return;
+        }
+        p_ = nullptr;
+    }
+    (void)hipGetLastError();
+    const hipError_t e = hipMalloc(&p_, bytes);
+    if (e != hipSuccess) {
+        p_ = nullptr;
+        (void)hipGetLastError();
+        throw AllocError("hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
+                         hipGetErrorString(e));
+    }
+    n_ = bytes;
+}
+
+void TempBuffer::reset() {
+    if (p_) {
+        if (pooled_)
+            (void)hipFreeAsync(p_, stream_);
+        else
+            (void)hipFree(p_);
+    }
+    p_ = nullptr;
+    n_ = 0;
+    stream_ = nullptr;
+    pooled_ = false;
 }
 
 void PinnedBuffer::reserve(size_t bytes) {

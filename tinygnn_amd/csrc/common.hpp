@@ -123,6 +123,39 @@ private:
     size_t n_ = 0;
 };
 
+// RAII device memory for a call's own temporaries, allocated and freed in
+// stream order from the library's pool of the current device: a call neither
+// waits for the GPU nor enters the driver once the pool is warm (hipMalloc and
+// hipFree of a 100 MB workspace on every call cost a SAGE-Max layer of 100K
+// nodes 5.3 of its 5.8 ms).  The pool keeps at most kPoolKeep freed bytes; the
+// rest goes back to the device at the next synchronisation, and all of it
+// before an allocation fails.  Where s is being captured the memory comes from
+// hipMalloc, which capture refuses.
+class TempBuffer {
+public:
+    TempBuffer() = default;
+    TempBuffer(size_t bytes, hipStream_t s) { allocate(bytes, s); }
+    ~TempBuffer() { reset(); }
+    TempBuffer(const TempBuffer&) = delete;
+    TempBuffer& operator=(const TempBuffer&) = delete;
+    void allocate(size_t bytes, hipStream_t s);  // discards contents
+    void reset();
+    // Frees on the null stream instead of s, for memory that outlives the call
+    // (s may be gone); the device must be idle by then.
+    void outlive_stream() { stream_ = nullptr; }
+    void* get() const { return p_; }
+    template <typename T> T* as() const { return static_cast<T*>(p_); }
+    size_t size() const { return n_; }
+    // false: hipMalloc memory; freeing it waits for the device
+    bool pooled() const { return pooled_; }
+
+private:
+    void* p_ = nullptr;
+    size_t n_ = 0;
+    hipStream_t stream_ = nullptr;
+    bool pooled_ = false;
+};
+
 // RAII pinned host allocation (hipHostMalloc): small device-to-host results
 // that the host reads after a stream synchronisation, so that the copies
 // themselves stay asynchronous.

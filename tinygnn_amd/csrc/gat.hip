@@ -1275,9 +1275,9 @@ void gat_aggregate(const tg_spmm_plan_s& p, int64_t n, int64_t heads, int64_t f,
     if (n == 0) return;
     if (p.n_split > 0)
         require(ftot <= p.max_f, "GATLayer: heads * f exceeds the plan's max_f");
-    DeviceBuffer own;
+    TempBuffer own;
     if (work == nullptr) {
-        own.resize(gat_ws_partials(p.n_partials, n, heads, f, concat));
+        own.allocate(gat_ws_partials(p.n_partials, n, heads, f, concat), s);
         work = own.get();
         work_bytes = own.size();
     }
@@ -1326,7 +1326,6 @@ void gat_aggregate(const tg_spmm_plan_s& p, int64_t n, int64_t heads, int64_t f,
             tmp, n, static_cast<int>(heads), static_cast<int>(f), out, ldo, post, exact ? 1 : 0);
         TG_LAUNCH_CHECK();
     }
-    if (own.get()) TG_HIP(hipStreamSynchronize(s));
 }
 
 bool gat_blocked_ok(int64_t heads, int64_t f, int concat) {

@@ -964,7 +964,7 @@ void sort_rows(int64_t n, const int32_t* row_ptr, int32_t* col, const int32_t* l
     probe.take<int64_t>(n_tiles);
     probe.take<int64_t>(n_tiles);
     probe.take<int32_t>(n_long);
-    DeviceBuffer buf(probe.bytes());
+    TempBuffer buf(probe.bytes(), s);
     Carver c(buf.get(), buf.size());
     int32_t* tmp = c.take<int32_t>(total);
     int64_t* d_seg = c.take<int64_t>(n_long + 1);
@@ -1035,9 +1035,9 @@ void self_loops_impl(bool norm, int64_t n, int64_t nnz, const int32_t* row_ptr,
     probe.take<float>(n);
     probe.take<int64_t>(scan_temp_elems(n));
     probe.take<int32_t>(n + 1);  // long-row list + its count
-    DeviceBuffer own;
+    TempBuffer own;
     if (workspace == nullptr) {
-        own.resize(probe.bytes());
+        own.allocate(probe.bytes(), s);
         workspace = own.get();
         ws_bytes = own.size();
     }
@@ -1080,7 +1080,6 @@ void self_loops_impl(bool norm, int64_t n, int64_t nnz, const int32_t* row_ptr,
                                        long_blocks, first_ins, row_ptr_out, dis, col_out,
                                        val_out);
     TG_LAUNCH_CHECK();
-    if (own.get()) TG_HIP(hipStreamSynchronize(s));  // own workspace is freed on return
 }
 
 size_t self_loops_ws(int64_t n) {
@@ -1113,9 +1112,9 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
     require(row_ptr != nullptr, W + ": row_ptr is null");
     require(n_edges == 0 || (src && dst && col_ind && val),
             W + ": null pointer");
-    DeviceBuffer own;
+    TempBuffer own;
     if (workspace == nullptr) {
-        own.resize(edge_list_to_csr_ws(n_nodes, n_edges));
+        own.allocate(edge_list_to_csr_ws(n_nodes, n_edges), s);
         workspace = own.get();
         ws_bytes = own.size();
     }
@@ -1140,7 +1139,6 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
         if (edge_sort_ready(h)) {
             edge_sort_finish(h, n_nodes, n_edges, src, dst, row_ptr, col_ind, val, workspace,
                              ws_bytes, s);
-            if (own.get()) TG_HIP(hipStreamSynchronize(s));
             return;
         }
     }
@@ -1170,7 +1168,6 @@ void edge_list_to_csr(int64_t n_nodes, int64_t n_edges, const int32_t* src, cons
         TG_LAUNCH_CHECK();
         sort_rows(n_nodes, row_ptr, col_ind, w.lists, counts, s);
     }
-    if (own.get()) TG_HIP(hipStreamSynchronize(s));
 }
 
 size_t edge_list_to_csr_ws(int64_t n_nodes, int64_t n_edges) {
@@ -1192,7 +1189,7 @@ void csr_validate(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t* ro
         throw std::invalid_argument("Tensor::sparse_csr: row_ptr.back() (" +
                                     std::to_string(static_cast<std::size_t>(last)) +
                                     ") must equal values.size() (" + std::to_string(nnz) + ")");
-    DeviceBuffer b(2 * sizeof(unsigned long long));
+    TempBuffer b(2 * sizeof(unsigned long long), s);
     auto* bad = b.as<unsigned long long>();
     fill_i32(reinterpret_cast<int32_t*>(bad), 4, -1, s);
     csr_check_kernel<<<grid_for(std::max(nnz, n_rows + 1), 256, 16384), 256, 0, s>>>(

@@ -56,17 +56,29 @@ struct CsvMeta {
 }  // namespace
 
 struct tg_csv_s {
-    tg::DeviceBuffer own_text;  // the file's bytes, when tg_csv_open read it
+    // The handle's memory outlives the stream of the call that made it: it is
+    // freed once the device is idle.
+    ~tg_csv_s() { (void)hipDeviceSynchronize(); }
+    static void make(tg::TempBuffer& b, size_t bytes, hipStream_t s) {
+        b.allocate(bytes, s);
+        b.outlive_stream();
+    }
+    tg::TempBuffer own_text;  // the file's bytes, when tg_csv_open read it
     const unsigned char* text = nullptr;
     int64_t n_bytes = 0;
     std::string name;
     int64_t n_lines = 0;
     int header = 0;
-    tg::DeviceBuffer lb, le;  // int64 [n_lines]
+    tg::TempBuffer bounds;  // int64 [2 n_lines]: lb, then le
+    int64_t* lb = nullptr;
+    int64_t* le = nullptr;
     tg::DeviceBuffer meta;    // CsvMeta
     tg::DeviceBuffer pow10;   // numparse::Pow10Entry [kPow10Count]
     // feature pass A, kept between tg_csv_feature_shape and the parse
-    tg::DeviceBuffer node, cnt, tok;  // int32 [n_data]
+    tg::TempBuffer fields;  // int32 [3 n_data]: node, cnt, tok
+    int32_t* node = nullptr;
+    int32_t* cnt = nullptr;
+    int32_t* tok = nullptr;
     bool shape_done = false;
     int64_t rows = 0, cols = 0;
 };
@@ -456,39 +468,51 @@ void index_lines(tg_csv_s& c, hipStream_t s) {
     const Granules gr = granules_of(c.text, c.n_bytes);
     const int64_t nb = ceil_div(gr.count, kIdxTileGranules);
     require(nb < (int64_t(1) << 31), "GraphLoader: file too large");
-    DeviceBuffer counts(sizeof(int32_t) * nb), offs(sizeof(int32_t) * (nb + 1));
-    DeviceBuffer temp(sizeof(int64_t) * scan_temp_elems(nb));
-    nl_count_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, counts.as<int32_t>(),
+    // (a free of pool memory costs up to 20 us of host time: few, whole pieces)
+    Carver p1(nullptr, 0);
+    p1.take<int32_t>(nb);
+    p1.take<int32_t>(nb + 1);
+    p1.take<int64_t>(scan_temp_elems(nb));
+    TempBuffer tiles(p1.bytes(), s);
+    Carver c1(tiles.get(), tiles.size());
+    int32_t* counts = c1.take<int32_t>(nb);
+    int32_t* offs = c1.take<int32_t>(nb + 1);
+    int64_t* temp = c1.take<int64_t>(scan_temp_elems(nb));
+    nl_count_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, counts,
                                                                      c.meta.as<CsvMeta>());
     TG_LAUNCH_CHECK();
     const int64_t n_nl = int64_t(read_meta(c, s).total_nl);
     if (n_nl >= (int64_t(1) << 31) - 2)
         throw std::runtime_error("GraphLoader: more than 2^31 lines in '" + c.name + "'");
-    exclusive_scan_i32(counts.as<int32_t>(), offs.as<int32_t>(), nb, temp.as<int64_t>(), s);
-    DeviceBuffer nl(sizeof(int64_t) * std::max<int64_t>(n_nl, 1));
-    nl_write_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, offs.as<int32_t>(),
-                                                                     nl.as<int64_t>());
-    TG_LAUNCH_CHECK();
+    exclusive_scan_i32(counts, offs, nb, temp, s);
     const int64_t n_seg = n_nl + 1;
-    DeviceBuffer flags(sizeof(int32_t) * n_seg), pos(sizeof(int32_t) * (n_seg + 1));
-    DeviceBuffer temp2(sizeof(int64_t) * scan_temp_elems(n_seg));
-    seg_flag_kernel<<<grid_of(n_seg, 256), 256, 0, s>>>(c.text, c.n_bytes, nl.as<int64_t>(), n_nl,
-                                                        flags.as<int32_t>());
+    Carver p2(nullptr, 0);
+    p2.take<int64_t>(n_seg);
+    p2.take<int32_t>(n_seg);
+    p2.take<int32_t>(n_seg + 1);
+    p2.take<int64_t>(scan_temp_elems(n_seg));
+    TempBuffer segs(p2.bytes(), s);
+    Carver c2(segs.get(), segs.size());
+    int64_t* nl = c2.take<int64_t>(n_seg);
+    int32_t* flags = c2.take<int32_t>(n_seg);
+    int32_t* pos = c2.take<int32_t>(n_seg + 1);
+    int64_t* temp2 = c2.take<int64_t>(scan_temp_elems(n_seg));
+    nl_write_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, offs, nl);
     TG_LAUNCH_CHECK();
-    exclusive_scan_i32(flags.as<int32_t>(), pos.as<int32_t>(), n_seg, temp2.as<int64_t>(), s);
-    c.lb.resize(sizeof(int64_t) * n_seg);
-    c.le.resize(sizeof(int64_t) * n_seg);
-    seg_write_kernel<<<grid_of(n_seg, 256), 256, 0, s>>>(c.text, c.n_bytes, nl.as<int64_t>(), n_nl,
-                                                         pos.as<int32_t>(), c.lb.as<int64_t>(),
-                                                         c.le.as<int64_t>());
+    seg_flag_kernel<<<grid_of(n_seg, 256), 256, 0, s>>>(c.text, c.n_bytes, nl, n_nl, flags);
     TG_LAUNCH_CHECK();
-    header_kernel<<<1, 1, 0, s>>>(c.text, c.lb.as<int64_t>(), c.le.as<int64_t>(),
-                                  pos.as<int32_t>() + n_seg, c.meta.as<CsvMeta>());
+    exclusive_scan_i32(flags, pos, n_seg, temp2, s);
+    c.make(c.bounds, 2 * sizeof(int64_t) * n_seg, s);
+    c.lb = c.bounds.as<int64_t>();
+    c.le = c.lb + n_seg;
+    seg_write_kernel<<<grid_of(n_seg, 256), 256, 0, s>>>(c.text, c.n_bytes, nl, n_nl, pos, c.lb,
+                                                         c.le);
+    TG_LAUNCH_CHECK();
+    header_kernel<<<1, 1, 0, s>>>(c.text, c.lb, c.le, pos + n_seg, c.meta.as<CsvMeta>());
     TG_LAUNCH_CHECK();
     int32_t n_lines = 0;
-    TG_HIP(hipMemcpyAsync(&n_lines, pos.as<int32_t>() + n_seg, sizeof n_lines,
-                          hipMemcpyDeviceToHost, s));
-    const CsvMeta m = read_meta(c, s);  // synchronises (the buffers above die here)
+    TG_HIP(hipMemcpyAsync(&n_lines, pos + n_seg, sizeof n_lines, hipMemcpyDeviceToHost, s));
+    const CsvMeta m = read_meta(c, s);  // synchronises
     c.n_lines = n_lines;
     c.header = m.header;
 }
@@ -496,8 +520,8 @@ void index_lines(tg_csv_s& c, hipStream_t s) {
 // The trimmed text of line i (for messages).
 std::string line_text(const tg_csv_s& c, int64_t i, hipStream_t s) {
     int64_t be[2];
-    TG_HIP(hipMemcpyAsync(&be[0], c.lb.as<int64_t>() + i, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    TG_HIP(hipMemcpyAsync(&be[1], c.le.as<int64_t>() + i, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    TG_HIP(hipMemcpyAsync(&be[0], c.lb + i, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    TG_HIP(hipMemcpyAsync(&be[1], c.le + i, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     TG_HIP(hipStreamSynchronize(s));
     std::string t(static_cast<size_t>(be[1] - be[0]), '\0');
     if (!t.empty())
@@ -526,7 +550,7 @@ void read_file(const char* path, tg_csv_s& c, hipStream_t s) {
     const int64_t n = static_cast<int64_t>(std::ftell(f));
     if (n < 0) throw std::runtime_error("GraphLoader: cannot read '" + p + "'");
     std::rewind(f);
-    c.own_text.resize(static_cast<size_t>(std::max<int64_t>(n, 1)));
+    c.make(c.own_text, static_cast<size_t>(std::max<int64_t>(n, 1)), s);
     constexpr size_t kStage = size_t(32) << 20;
     void* stage[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};
@@ -567,16 +591,16 @@ void feature_shape(tg_csv_s& c, hipStream_t s) {
     const int64_t n_data = c.n_lines - c.header;
     if (n_data == 0)
         throw std::runtime_error("GraphLoader::parse_features: no data rows in '" + c.name + "'");
-    c.node.resize(sizeof(int32_t) * n_data);
-    c.cnt.resize(sizeof(int32_t) * n_data);
-    c.tok.resize(sizeof(int32_t) * n_data);
+    c.make(c.fields, 3 * sizeof(int32_t) * n_data, s);
+    c.node = c.fields.as<int32_t>();
+    c.cnt = c.node + n_data;
+    c.tok = c.cnt + n_data;
     reset_meta(c, s);
     feat_a_kernel<<<static_cast<unsigned>(n_data), kWave, 0, s>>>(
-        c.text, c.lb.as<int64_t>(), c.le.as<int64_t>(), c.header, c.node.as<int32_t>(),
-        c.cnt.as<int32_t>(), c.meta.as<CsvMeta>());
+        c.text, c.lb, c.le, c.header, c.node, c.cnt, c.meta.as<CsvMeta>());
     TG_LAUNCH_CHECK();
     int32_t first_cnt = 0;
-    TG_HIP(hipMemcpyAsync(&first_cnt, c.cnt.get(), sizeof first_cnt, hipMemcpyDeviceToHost, s));
+    TG_HIP(hipMemcpyAsync(&first_cnt, c.cnt, sizeof first_cnt, hipMemcpyDeviceToHost, s));
     const CsvMeta m = read_meta(c, s);
     c.rows = int64_t(m.max_id) + 1;
     c.cols = std::max<int32_t>(first_cnt, 0);
@@ -647,8 +671,8 @@ int tg_csv_parse_edges(tg_csv_t csv, int32_t* src, int32_t* dst, int64_t* max_id
         tg::reset_meta(*csv, s);
         if (n_data > 0) {
             tg::edges_kernel<<<tg::grid_of(n_data, 256), 256, 0, s>>>(
-                csv->text, csv->lb.as<int64_t>(), csv->le.as<int64_t>(), csv->header, n_data,
-                src, dst, csv->meta.as<CsvMeta>());
+                csv->text, csv->lb, csv->le, csv->header, n_data, src, dst,
+                csv->meta.as<CsvMeta>());
             TG_LAUNCH_CHECK();
         }
         const CsvMeta m = tg::read_meta(*csv, s);
@@ -695,9 +719,9 @@ int tg_csv_parse_features(tg_csv_t csv, float* out, int64_t n_rows, int64_t ld,
         require(ld >= cols, "GraphLoader::parse_features: ld below the table's columns");
         require(out != nullptr || n_rows * cols == 0, "GraphLoader::parse_features: null output");
         const int64_t n_data = csv->n_lines - csv->header;
-        tg::DeviceBuffer winner(sizeof(int32_t) * std::max<int64_t>(rows, 1));
+        tg::TempBuffer winner(sizeof(int32_t) * std::max<int64_t>(rows, 1), s);
         tg::fill_i32(winner.as<int32_t>(), rows, -1, s);
-        tg::winner_kernel<<<tg::grid_of(n_data, 256), 256, 0, s>>>(csv->node.as<int32_t>(), n_data,
+        tg::winner_kernel<<<tg::grid_of(n_data, 256), 256, 0, s>>>(csv->node, n_data,
                                                                   winner.as<int32_t>());
         TG_LAUNCH_CHECK();
         if (n_rows * cols > 0) {
@@ -708,12 +732,11 @@ int tg_csv_parse_features(tg_csv_t csv, float* out, int64_t n_rows, int64_t ld,
         }
         tg::reset_meta(*csv, s);
         tg::feat_b_kernel<<<static_cast<unsigned>(n_data), tg::kWave, 0, s>>>(
-            csv->text, csv->lb.as<int64_t>(), csv->le.as<int64_t>(), csv->header,
-            csv->node.as<int32_t>(), csv->cnt.as<int32_t>(), winner.as<int32_t>(),
-            csv->pow10.as<tg::numparse::Pow10Entry>(), ld, out, csv->tok.as<int32_t>(),
+            csv->text, csv->lb, csv->le, csv->header, csv->node, csv->cnt, winner.as<int32_t>(),
+            csv->pow10.as<tg::numparse::Pow10Entry>(), ld, out, csv->tok,
             csv->meta.as<CsvMeta>());
         TG_LAUNCH_CHECK();
-        const CsvMeta m = tg::read_meta(*csv, s);  // synchronises; winner dies after
+        const CsvMeta m = tg::read_meta(*csv, s);  // synchronises
         if (m.first_err == ~0ull) return;
         const int64_t i = static_cast<int64_t>(m.first_err >> 3);
         const int64_t d = i - csv->header;
@@ -728,12 +751,12 @@ int tg_csv_parse_features(tg_csv_t csv, float* out, int64_t n_rows, int64_t ld,
                                      tg::field_of(line, 0) + "'");
         if (code == tg::kErrInvalidFeature) {
             int32_t t = 0;
-            TG_HIP(hipMemcpy(&t, csv->tok.as<int32_t>() + d, 4, hipMemcpyDeviceToHost));
+            TG_HIP(hipMemcpy(&t, csv->tok + d, 4, hipMemcpyDeviceToHost));
             throw std::runtime_error(P + "invalid feature on line " + ln + ": '" +
                                      tg::field_of(line, t) + "'");
         }
         int32_t got = 0;
-        TG_HIP(hipMemcpy(&got, csv->cnt.as<int32_t>() + d, 4, hipMemcpyDeviceToHost));
+        TG_HIP(hipMemcpy(&got, csv->cnt + d, 4, hipMemcpyDeviceToHost));
         throw std::runtime_error(P + "inconsistent feature count on line " + ln + ": expected " +
                                  std::to_string(cols) + " but got " + std::to_string(got));
     });

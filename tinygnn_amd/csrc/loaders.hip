@@ -230,7 +230,7 @@ int tg_cora_upload(tg_cora_t c, float* features, int32_t* row_ptr, int32_t* col_
             TG_HIP(hipMemcpyAsync(features, c->features.data(),
                                   static_cast<size_t>(c->n * c->f) * sizeof(float),
                                   hipMemcpyHostToDevice, s));
-        tg::DeviceBuffer edges(static_cast<size_t>(std::max<int64_t>(c->e, 1)) * 8);
+        tg::TempBuffer edges(static_cast<size_t>(std::max<int64_t>(c->e, 1)) * 8, s);
         int32_t* d_src = edges.as<int32_t>();
         int32_t* d_dst = d_src + c->e;
         if (c->e > 0) {

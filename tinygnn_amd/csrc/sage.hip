@@ -121,9 +121,9 @@ void sage_forward(const tg_spmm_plan_s& p, int64_t n, int64_t f_in, int64_t f_ou
             "SAGELayer: unknown dataflow");
     require(dataflow == TG_SAGE_CONCAT || agg == TG_AGG_MEAN,
             "SAGELayer: transform-first needs the mean aggregator");
-    DeviceBuffer own;
+    TempBuffer own;
     if (work == nullptr) {
-        own.resize(sage_ws(n, f_in, f_out, dataflow));
+        own.allocate(sage_ws(n, f_in, f_out, dataflow), s);
         work = own.get();
         work_bytes = own.size();
     }
@@ -205,7 +205,6 @@ void sage_forward(const tg_spmm_plan_s& p, int64_t n, int64_t f_in, int64_t f_ou
             run_aggregate(p, f_out, ci, nullptr, t + fp, 2 * fp, out, f_out, epi, s);
         }
     }
-    if (own.get()) TG_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace tg
