@@ -147,6 +147,40 @@ def test_long_lines(gpu, restate):
     assert _gpu_feats(gpu, short) == _ora_feats(restate, short)
 
 
+@pytest.mark.parametrize("offset", [0, 1, 15])
+def test_short_field_paths(gpu, restate, offset):
+    """Edge lines and feature fields around the limits of the conversions in
+    registers (16 bytes, 9 digits, signs, points, float midpoints) and around
+    the ends of the feature parser's 1 KB windows, at the end of the text."""
+    edges = ["1,2", "0,0", "007,123456789", "123456789,987654321", "1234567890,1", "1,1234567890",
+             "12345678,1234567", "12345678,12345678", "+5,6", "5,+6", "5,6 junk", "5 ,6", "0,1",
+             "12345678,123456x", "3,4"]
+    text = ("\n".join(edges)).encode()
+    assert _gpu_edges(gpu, text, offset=offset) == _ora_edges(restate, text)
+    for bad in ("1,2,3", "1;2", "4,", ",4", "-1,4", "4,-1", "99999999999,1"):
+        t = ("1,2\n" + bad + "\n3,4").encode()
+        assert _gpu_edges(gpu, t, offset=offset) == _ora_edges(restate, t)
+    fields = ["1", "-1", "+1", " 1", "  1", "-0", "0.0", ".5", "-.5", "5.", "-", ".", "1.5x", "1e3",
+              "0.000000001", "123456789", "1234567890", "12345.6789", "-1234567.89", "16777217",
+              "16777217.0", "16777219", "-33554434.5", "33554435", "9.99999999", "1.000000059",
+              "0.1234567890123", "0.12345678901234", "1_", "0x1p3", "inf", "1 2", "000000001",
+              "0000000012", "-123456.7890123456"]
+    for f in fields:  # one by one: some are errors
+        t = ("0," + f + ",2.5\n1,1.25," + f + "\n").encode()
+        assert _gpu_feats(gpu, t, offset=offset) == _ora_feats(restate, t), f
+    rng = np.random.default_rng(5)
+    for total in (1008, 1023, 1024, 1025, 2047, 2048, 2049, 3100):
+        for tail in ("", ","):
+            row = "0"
+            while len(row) < total - 12:
+                row += ",%.6f" % (rng.random() * 20 - 10)
+            row += "," + "7" * (total - len(row) - 1 - len(tail)) + tail
+            assert len(row) == total
+            n = row.count(",") - len(tail)
+            t = (row + "\n1" + ",0.5" * n + "\n").encode()
+            assert _gpu_feats(gpu, t, offset=offset) == _ora_feats(restate, t), (total, tail)
+
+
 def test_large_files(gpu, restate, tmp_path):
     """Millions of edge lines and a 30,000 x 100 feature table through the
     file path (pinned staging, overlapped copies), then a planted defect near

@@ -16,14 +16,16 @@
 //   3. The header test (is_header, :24-33) on line 0.
 //   4. Edges: one thread per line, the first comma, then std::stoi of both
 //      sides (:73-99).
-//   5. Features: one wavefront per line.
-//      * Pass A counts the fields (std::getline semantics: a trailing comma
-//        yields no last field) and parses node_id.
+//   5. Features.
+//      * Pass A parses every line's node_id, and counts the first line's
+//        fields (std::getline semantics: a trailing comma yields no last
+//        field).
 //      * The last line of every node_id is marked; earlier ones are
 //        overwritten in the reference (:191-197).
-//      * Pass B finds the commas 1 KB at a time (16 B per lane; positions
-//        compacted in LDS), and each lane converts whole fields with
-//        std::stof's semantics (numparse.hpp), writing the marked lines' rows.
+//      * Pass B, one wavefront per line, finds the commas 1 KB at a time
+//        (16 B per lane; text and positions in LDS), and each lane converts
+//        whole fields with std::stof's semantics (short decimals by one exact
+//        division, the rest by numparse.hpp), writing the marked lines' rows.
 //
 // Errors: every line computes its own error code.  An atomic minimum over
 // (line << 3 | code) selects the first, which is the one the reference's
@@ -48,17 +50,26 @@ namespace {
 
 struct CsvMeta {
     unsigned long long first_err;  // (line << 3) | code; ~0 when none
-    unsigned long long total_nl;   // newline count
     int32_t max_id;                // largest endpoint / node_id, -1 if none
     int32_t header;
+    int32_t n_lines;
+    int32_t first_cnt;             // feature fields of the first data line
 };
 
 }  // namespace
 
 struct tg_csv_s {
     // The handle's memory outlives the stream of the call that made it: it is
-    // freed once the device is idle.
-    ~tg_csv_s() { (void)hipDeviceSynchronize(); }
+    // freed once its device is idle.
+    tg_csv_s() { (void)hipGetDevice(&device); }
+    ~tg_csv_s() {
+        int now = device;
+        (void)hipGetDevice(&now);
+        if (now != device) (void)hipSetDevice(device);
+        (void)hipDeviceSynchronize();
+        if (now != device) (void)hipSetDevice(now);
+    }
+    int device = 0;
     static void make(tg::TempBuffer& b, size_t bytes, hipStream_t s) {
         b.allocate(bytes, s);
         b.outlive_stream();
@@ -154,13 +165,13 @@ Granules granules_of(const unsigned char* text, int64_t n) {
 
 __global__ void meta_init_kernel(CsvMeta* m) {
     m->first_err = ~0ull;
-    m->total_nl = 0;
     m->max_id = -1;
     m->header = 0;
+    m->n_lines = 0;
+    m->first_cnt = 0;
 }
 
-__global__ __launch_bounds__(kIdxBlock) void nl_count_kernel(Granules gr, int32_t* counts,
-                                                             CsvMeta* meta) {
+__global__ __launch_bounds__(kIdxBlock) void nl_count_kernel(Granules gr, int32_t* counts) {
     __shared__ int32_t red[kIdxBlock / kWave];
     int c = 0;
     for (int r = 0; r < kIdxRounds; ++r) {
@@ -174,7 +185,6 @@ __global__ __launch_bounds__(kIdxBlock) void nl_count_kernel(Granules gr, int32_
         int t = 0;
         for (int w = 0; w < kIdxBlock / kWave; ++w) t += red[w];
         counts[blockIdx.x] = t;
-        if (t) atomicAdd(&meta->total_nl, static_cast<unsigned long long>(t));
     }
 }
 
@@ -248,90 +258,162 @@ __global__ void header_kernel(const unsigned char* text, const int64_t* lb, cons
         }
     }
     meta->header = h;
+    meta->n_lines = *n_lines;
 }
 
 __device__ __forceinline__ void record_error(CsvMeta* meta, int64_t line, int code) {
     atomicMin(&meta->first_err, (static_cast<unsigned long long>(line) << 3) | unsigned(code));
 }
 
-__device__ __forceinline__ void block_max_id(int v, CsvMeta* meta) {
-    // one atomic per wavefront
-    v = max(v, __shfl_xor(v, 32, kWave));
-    v = max(v, __shfl_xor(v, 16, kWave));
-    v = max(v, __shfl_xor(v, 8, kWave));
-    v = max(v, __shfl_xor(v, 4, kWave));
-    v = max(v, __shfl_xor(v, 2, kWave));
-    v = max(v, __shfl_xor(v, 1, kWave));
-    if ((threadIdx.x & (kWave - 1)) == 0 && v >= 0) atomicMax(&meta->max_id, v);
+// Raises meta->max_id to v.  The value in memory is looked at first: of N ids in
+// any order but ascending few are new maxima, and an atomic per wavefront on one
+// address was all that the parsers waited for (78,000 of them 0.9 ms).
+__device__ __forceinline__ void raise_max_id(int v, CsvMeta* meta) {
+    if (v > __hip_atomic_load(&meta->max_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&meta->max_id, v);
 }
 
+// Raises meta->max_id to the workgroup's largest v (256 threads, all of them).
+__device__ __forceinline__ void block_max_id(int v, CsvMeta* meta) {
+    __shared__ int best[256 / kWave];
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
+    if ((threadIdx.x & (kWave - 1)) == 0) best[threadIdx.x / kWave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 256 / kWave; ++w) v = max(v, best[w]);
+        if (v >= 0) raise_max_id(v, meta);
+    }
+}
+
+// The 16 bytes from byte `sh` (0 to 3) of the five words at q, as four words.
+__device__ __forceinline__ void load16(const uint32_t* q, uint32_t sh, uint32_t (&w)[4]) {
+    uint32_t x[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) x[k] = q[k];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_alignbyte(x[k + 1], x[k], sh);
+}
+
+__device__ __forceinline__ uint32_t byte_of(const uint32_t (&w)[4], int i) {
+    return (w[i / 4] >> (8 * (i % 4))) & 0xFFu;
+}
+
+// "digits,digits" of at most 16 bytes, 1 to 9 digits a side, in registers:
+// false for any other line.
+__device__ __forceinline__ bool fast_edge(const unsigned char* p, int len, int32_t* s,
+                                          int32_t* t) {
+    uint32_t w[4];
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+    load16(reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3)), static_cast<uint32_t>(a & 3), w);
+    uint32_t v = 0, first = 0;
+    int digits = 0, first_digits = -1;
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (i < len) {
+            const uint32_t c = byte_of(w, i);
+            if (c == ',' && first_digits < 0) {
+                first = v;
+                first_digits = digits;
+                v = 0;
+                digits = 0;
+            } else {
+                ok = ok && c - '0' < 10u;
+                v = v * 10u + (c - '0');
+                ++digits;
+            }
+        }
+    }
+    *s = static_cast<int32_t>(first);
+    *t = static_cast<int32_t>(v);
+    return ok && first_digits >= 1 && first_digits <= 9 && digits >= 1 && digits <= 9;
+}
+
+// Workgroups of the kernels that take a line per thread or wavefront: enough
+// to fill the chip, and few enough that one atomic each for the largest id
+// costs nothing (ids in ascending order raise it every time).
+constexpr int64_t kLineGroups = 2048;
+
 // GraphLoader::parse_edges (graph_loader.cpp:61-107), one thread per line.
-__global__ __launch_bounds__(256) void edges_kernel(const unsigned char* text, const int64_t* lb,
-                                                    const int64_t* le, int64_t start,
-                                                    int64_t n_data, int32_t* src, int32_t* dst,
-                                                    CsvMeta* meta) {
-    const int64_t d = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// 5M lines of 12 bytes: 5 loads of a line into registers and no loop over its
+// bytes in memory; 109 us with byte loads (and 0.9 ms with an atomic per
+// wavefront for the largest id).
+__global__ __launch_bounds__(256) void edges_kernel(const unsigned char* text, int64_t n_bytes,
+                                                    const int64_t* lb, const int64_t* le,
+                                                    int64_t start, int64_t n_data, int32_t* src,
+                                                    int32_t* dst, CsvMeta* meta) {
     int best = -1;
-    if (d < n_data) {
+    for (int64_t d = int64_t(blockIdx.x) * 256 + threadIdx.x; d < n_data;
+         d += int64_t(gridDim.x) * 256) {
         const int64_t i = start + d;
         const int64_t b = lb[i], e = le[i];
-        int64_t c = b;
-        while (c < e && text[c] != ',') ++c;
         int32_t s = 0, t = 0;
-        int err = kErrNone;
-        if (c == e) {
-            err = kErrMalformed;
+        // (the loads of load16 end at most 20 bytes after b)
+        if (e - b > 16 || b + 20 > n_bytes || !fast_edge(text + b, int(e - b), &s, &t)) {
+            s = t = 0;
+            int64_t c = b;
+            while (c < e && text[c] != ',') ++c;
+            int err = kErrNone;
+            if (c == e) {
+                err = kErrMalformed;
+            } else {
+                const int r1 = np::parse_int(text + b, text + c, &s);
+                const int r2 = np::parse_int(text + c + 1, text + e, &t);
+                if (r1 != np::kOk || r2 != np::kOk) err = kErrInvalidInt;
+                else if (s < 0 || t < 0) err = kErrNegative;
+            }
+            if (err) {
+                record_error(meta, i, err);
+            } else {
+                best = max(best, max(s, t));
+            }
         } else {
-            const int r1 = np::parse_int(text + b, text + c, &s);
-            const int r2 = np::parse_int(text + c + 1, text + e, &t);
-            if (r1 != np::kOk || r2 != np::kOk) err = kErrInvalidInt;
-            else if (s < 0 || t < 0) err = kErrNegative;
+            best = max(best, max(s, t));
         }
         src[d] = s;
         dst[d] = t;
-        if (err) record_error(meta, i, err);
-        else best = max(s, t);
     }
     block_max_id(best, meta);
 }
 
-// Feature pass A (graph_loader.cpp:118-170): one wavefront per line counts
-// the fields and parses node_id.  node[d] = node_id, or -1 (invalid) / -2
-// (negative); cnt[d] = number of feature fields.
-__global__ __launch_bounds__(kWave) void feat_a_kernel(const unsigned char* text,
-                                                       const int64_t* lb, const int64_t* le,
-                                                       int64_t start, int32_t* node,
-                                                       int32_t* cnt, CsvMeta* meta) {
-    const int64_t d = blockIdx.x;
-    const int64_t i = start + d;
-    const int lane = threadIdx.x;
-    const int64_t b = lb[i], e = le[i];
-    const uintptr_t base = reinterpret_cast<uintptr_t>(text);
-    const uintptr_t a_first = (base + b) & ~uintptr_t(15);
-    const uintptr_t a_end = base + e;
-    int commas = 0;
-    for (uintptr_t a = a_first + 16 * lane; a < a_end; a += 16 * kWave) {
-        const uint4 v = *reinterpret_cast<const uint4*>(a);
-        const int64_t off = int64_t(a - base);
-        commas += __popc(eq16(v, 0x2c2c2c2cu) & range16(b - off, e - off));
+// Feature pass A (graph_loader.cpp:118-170): node_id of every line, one thread
+// per line, node[d] = node_id, or -1 (invalid) / -2 (negative); the first
+// workgroup counts the first line's feature fields.  (Counting every line's
+// here too read the whole text once more: 0.1 ms for 100 MB.)
+__global__ __launch_bounds__(256) void feat_a_kernel(const unsigned char* text,
+                                                     const int64_t* lb, const int64_t* le,
+                                                     int64_t start, int64_t n_data, int32_t* node,
+                                                     CsvMeta* meta) {
+    if (blockIdx.x == 0) {
+        __shared__ int total;
+        if (threadIdx.x == 0) total = 0;
+        __syncthreads();
+        const int64_t b = lb[start], e = le[start];
+        const uintptr_t base = reinterpret_cast<uintptr_t>(text);
+        int commas = 0;
+        for (uintptr_t a = ((base + b) & ~uintptr_t(15)) + 16 * threadIdx.x; a < base + e;
+             a += 16 * 256) {
+            const uint4 v = *reinterpret_cast<const uint4*>(a);
+            const int64_t off = int64_t(a - base);
+            commas += __popc(eq16(v, 0x2c2c2c2cu) & range16(b - off, e - off));
+        }
+        if (commas) atomicAdd(&total, commas);
+        __syncthreads();
+        if (threadIdx.x == 0) meta->first_cnt = total - (text[e - 1] == ',' ? 1 : 0);
     }
-    commas = wave_sum(commas);
-    if (lane == 0) {
-        const int fields = commas + 1 - (text[e - 1] == ',' ? 1 : 0);
-        cnt[d] = fields - 1;
+    int best = -1;
+    for (int64_t d = int64_t(blockIdx.x) * 256 + threadIdx.x; d < n_data;
+         d += int64_t(gridDim.x) * 256) {
+        const int64_t b = lb[start + d], e = le[start + d];
         int64_t c = b;
         while (c < e && text[c] != ',') ++c;
         int32_t id = 0;
         const int r = np::parse_int(text + b, text + c, &id);
-        if (r != np::kOk) {
-            node[d] = -1;
-        } else if (id < 0) {
-            node[d] = -2;
-        } else {
-            node[d] = id;
-            atomicMax(&meta->max_id, id);
-        }
+        node[d] = r != np::kOk ? -1 : id < 0 ? -2 : id;
+        if (r == np::kOk) best = max(best, id);
     }
+    block_max_id(best, meta);
 }
 
 __global__ __launch_bounds__(256) void winner_kernel(const int32_t* node, int64_t n_data,
@@ -353,76 +435,138 @@ __global__ __launch_bounds__(256) void zero_rows_kernel(const int32_t* winner, i
     }
 }
 
-// Feature pass B (graph_loader.cpp:150-168,185-197), one wavefront per line.
-constexpr int kWindow = 16 * kWave;  // bytes per step
-
-__global__ __launch_bounds__(kWave) void feat_b_kernel(
-    const unsigned char* text, const int64_t* lb, const int64_t* le, int64_t start,
-    const int32_t* node, const int32_t* cnt, const int32_t* winner,
-    const np::Pow10Entry* pow10, int64_t ld, float* out, int32_t* tok, CsvMeta* meta) {
-    __shared__ int32_t cpos[kWindow];
-    const int64_t d = blockIdx.x;
-    const int64_t i = start + d;
-    const int lane = threadIdx.x;
-    const int64_t b = lb[i], e = le[i];
-    const int32_t id = node[d];
-    const int32_t my_cnt = cnt[d];
-    const int32_t expected = cnt[0];
-    const bool writable = id >= 0 && winner[id] == int32_t(d) && my_cnt == expected;
-    const uintptr_t base = reinterpret_cast<uintptr_t>(text);
-    const uintptr_t a_end = base + e;
-    int64_t carry = b;     // start of the field in progress
-    int64_t t0 = 0;        // index of the field ending at the window's first comma
-    int bad = 0x7fffffff;  // first field that fails to convert
-    auto convert = [&](int64_t fs, int64_t fe, int64_t t) {
-        if (t < 1) return;  // field 0 is node_id (pass A)
-        uint32_t bits;
-        const int r = np::parse_float(text + fs, text + fe, pow10, &bits);
-        if (r != np::kOk) {
-            bad = min(bad, int(t));
-        } else if (writable) {
-            out[int64_t(id) * ld + (t - 1)] = __uint_as_float(bits);
+// std::stof of a field "[sign or space] digits [. digits]" of at most 16 bytes
+// and 9 digits at byte `at` of a window in LDS (20 bytes readable): the digits
+// as an integer over a power of ten, both exact in double, so the double
+// quotient is the value rounded once, and its rounding to float is strtof's
+// unless the quotient is a float midpoint.  False, for the general conversion,
+// there and for any other field.
+__device__ __forceinline__ bool fast_float(const uint32_t* win, int at, int len, uint32_t* bits) {
+    if (len <= 0 || len > 16) return false;
+    uint32_t w[4];
+    load16(win + at / 4, static_cast<uint32_t>(at) & 3, w);
+    const uint32_t c0 = byte_of(w, 0);
+    const bool lead = c0 == '-' || c0 == '+' || c0 == ' ';
+    uint32_t v = 0;
+    int digits = 0, frac = 0;
+    bool ok = true, point = false;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (i < len && !(i == 0 && lead)) {
+            const uint32_t c = byte_of(w, i);
+            if (c == '.' && !point) {
+                point = true;
+            } else {
+                ok = ok && c - '0' < 10u;
+                v = v * 10u + (c - '0');
+                ++digits;
+                frac += point ? 1 : 0;
+            }
         }
-    };
-    for (uintptr_t w = (base + b) & ~uintptr_t(15); w < a_end; w += kWindow) {
-        const uintptr_t a = w + 16 * lane;
-        uint32_t m = 0;
-        if (a < a_end) {
-            const uint4 v = *reinterpret_cast<const uint4*>(a);
-            const int64_t off = int64_t(a - base);
-            m = eq16(v, 0x2c2c2c2cu) & range16(b - off, e - off);
-        }
-        const int c = __popc(m);
-        const int incl = wave_inclusive_scan(c);
-        const int k_total = __shfl(incl, kWave - 1, kWave);
-        int p = incl - c;
-        while (m) {
-            const int j = __ffs(m) - 1;
-            m &= m - 1;
-            cpos[p++] = int32_t(16 * lane + j);  // offset from w
-        }
-        __syncthreads();
-        const int64_t wo = int64_t(w - base);
-        for (int j = lane; j < k_total; j += kWave) {
-            const int64_t fs = j == 0 ? carry : wo + cpos[j - 1] + 1;
-            convert(fs, wo + cpos[j], t0 + j);
-        }
-        if (k_total > 0) carry = wo + cpos[k_total - 1] + 1;
-        t0 += k_total;
-        __syncthreads();
     }
-    if (lane == 0 && carry < e) convert(carry, e, t0);  // the last field
-    for (int s = kWave / 2; s > 0; s >>= 1) bad = min(bad, __shfl_xor(bad, s, kWave));
-    if (lane == 0) {
-        int err = kErrNone;
-        if (id == -1) err = kErrInvalidNode;
-        else if (id == -2) err = kErrNegativeNode;
-        else if (bad != 0x7fffffff) err = kErrInvalidFeature;
-        else if (d == 0 && my_cnt == 0) err = kErrNoFeatures;
-        else if (my_cnt != expected) err = kErrInconsistent;
-        if (err) {
-            tok[d] = bad;
-            record_error(meta, i, err);
+    if (!ok || digits < 1 || digits > 9) return false;
+    const double ten = ((frac & 1) ? 10.0 : 1.0) * ((frac & 2) ? 100.0 : 1.0) *
+                       ((frac & 4) ? 1e4 : 1.0) * ((frac & 8) ? 1e8 : 1.0);
+    const double q = static_cast<double>(v) / ten;
+    if ((static_cast<uint32_t>(__double_as_longlong(q)) & 0x1FFFFFFFu) == 0x10000000u)
+        return false;
+    *bits = __float_as_uint(static_cast<float>(q)) | (c0 == '-' ? 0x80000000u : 0u);
+    return true;
+}
+
+// Feature pass B (graph_loader.cpp:150-168,185-197), one wavefront per line:
+// its text a window of 1 KB at a time in LDS, its commas compacted there, a
+// field per lane converted from there.  cnt[d] = the line's feature fields.
+// 100,000 lines of 100 fields (100 MB) took 508 us with a wavefront per
+// workgroup and the fields' bytes read from memory one at a time.
+constexpr int kWindow = 16 * kWave;  // bytes per step
+constexpr int kFeatWaves = 4;
+
+__global__ __launch_bounds__(kFeatWaves * kWave) void feat_b_kernel(
+    const unsigned char* text, const int64_t* lb, const int64_t* le, int64_t start,
+    int64_t n_data, const int32_t* node, int32_t* cnt, int32_t expected, const int32_t* winner,
+    const np::Pow10Entry* pow10, int64_t ld, float* out, int32_t* tok, CsvMeta* meta) {
+    __shared__ __attribute__((aligned(16))) uint32_t windows[kFeatWaves][kWindow / 4 + 8];
+    __shared__ uint16_t commas[kFeatWaves][kWindow + 2];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    uint32_t* win = windows[wave];
+    uint16_t* cpos = commas[wave];
+    const uintptr_t base = reinterpret_cast<uintptr_t>(text);
+    for (int64_t d = int64_t(blockIdx.x) * kFeatWaves + wave; d < n_data;
+         d += int64_t(gridDim.x) * kFeatWaves) {
+        const int64_t i = start + d;
+        const int64_t b = lb[i], e = le[i];
+        const int32_t id = node[d];
+        const bool writable = id >= 0 && winner[id] == int32_t(d);
+        const uintptr_t a_end = base + e;
+        int64_t carry = b;     // start of the field in progress
+        int64_t t0 = 0;        // index of the field ending at the window's first comma
+        int bad = 0x7fffffff;  // first field that fails to convert
+        for (uintptr_t w = (base + b) & ~uintptr_t(15); w < a_end; w += kWindow) {
+            const uintptr_t a = w + 16 * lane;
+            const int64_t wo = int64_t(w - base);
+            uint32_t m = 0;
+            if (a < a_end) {
+                const uint4 v = *reinterpret_cast<const uint4*>(a);
+                const int64_t off = int64_t(a - base);
+                m = eq16(v, 0x2c2c2c2cu) & range16(b - off, e - off);
+                *reinterpret_cast<uint4*>(win + 4 * lane) = v;
+            }
+            const int c = __popc(m);
+            const int incl = wave_inclusive_scan(c);
+            int k_total = __shfl(incl, kWave - 1, kWave);
+            int p = incl - c;
+            while (m) {
+                const int j = __ffs(m) - 1;
+                m &= m - 1;
+                cpos[p++] = static_cast<uint16_t>(16 * lane + j);  // offset from w
+            }
+            // the window's text and commas, this wavefront's own
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            int64_t next = k_total > 0 ? wo + cpos[k_total - 1] + 1 : carry;
+            if (w + kWindow >= a_end && next < e) {  // the line's last field ends at e
+                if (lane == 0) cpos[k_total] = static_cast<uint16_t>(e - wo);
+                ++k_total;
+                next = e;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+            for (int j = lane; j < k_total; j += kWave) {
+                const int64_t t = t0 + j;
+                if (t < 1) continue;  // field 0 is node_id (pass A)
+                const int64_t fs = j == 0 ? carry : wo + cpos[j - 1] + 1;
+                const int64_t fe = wo + cpos[j];
+                uint32_t bits;
+                if (fs < wo || !fast_float(win, int(fs - wo), int(fe - fs), &bits)) {
+                    if (np::parse_float(text + fs, text + fe, pow10, &bits) != np::kOk) {
+                        bad = min(bad, int(t));
+                        continue;
+                    }
+                }
+                if (writable && t <= expected)
+                    out[int64_t(id) * ld + (t - 1)] = __uint_as_float(bits);
+            }
+            carry = next;
+            t0 += k_total;
+            // (read before the next window overwrites them)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        for (int s = kWave / 2; s > 0; s >>= 1) bad = min(bad, __shfl_xor(bad, s, kWave));
+        if (lane == 0) {
+            const int32_t my_cnt = int32_t(t0) - 1;
+            cnt[d] = my_cnt;
+            int err = kErrNone;
+            if (id == -1) err = kErrInvalidNode;
+            else if (id == -2) err = kErrNegativeNode;
+            else if (bad != 0x7fffffff) err = kErrInvalidFeature;
+            else if (d == 0 && my_cnt == 0) err = kErrNoFeatures;
+            else if (my_cnt != expected) err = kErrInconsistent;
+            if (err) {
+                tok[d] = bad;
+                record_error(meta, i, err);
+            }
         }
     }
 }
@@ -454,6 +598,10 @@ void reset_meta(tg_csv_s& c, hipStream_t s) {
 
 unsigned grid_of(int64_t n, int block) { return static_cast<unsigned>(ceil_div(n, block)); }
 
+unsigned line_groups(int64_t n, int block) {
+    return static_cast<unsigned>(std::min(ceil_div(n, block), kLineGroups));
+}
+
 void index_lines(tg_csv_s& c, hipStream_t s) {
     c.meta.resize(sizeof(CsvMeta));
     c.pow10.resize(sizeof(np::Pow10Entry) * np::kPow10Count);
@@ -468,7 +616,6 @@ void index_lines(tg_csv_s& c, hipStream_t s) {
     const Granules gr = granules_of(c.text, c.n_bytes);
     const int64_t nb = ceil_div(gr.count, kIdxTileGranules);
     require(nb < (int64_t(1) << 31), "GraphLoader: file too large");
-    // (a free of pool memory costs up to 20 us of host time: few, whole pieces)
     Carver p1(nullptr, 0);
     p1.take<int32_t>(nb);
     p1.take<int32_t>(nb + 1);
@@ -478,13 +625,16 @@ void index_lines(tg_csv_s& c, hipStream_t s) {
     int32_t* counts = c1.take<int32_t>(nb);
     int32_t* offs = c1.take<int32_t>(nb + 1);
     int64_t* temp = c1.take<int64_t>(scan_temp_elems(nb));
-    nl_count_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, counts,
-                                                                     c.meta.as<CsvMeta>());
+    nl_count_kernel<<<static_cast<unsigned>(nb), kIdxBlock, 0, s>>>(gr, counts);
     TG_LAUNCH_CHECK();
-    const int64_t n_nl = int64_t(read_meta(c, s).total_nl);
+    exclusive_scan_i32(counts, offs, nb, temp, s);
+    // the scan's 64-bit total (offs wraps past 2^31)
+    int64_t n_nl = 0;
+    TG_HIP(hipMemcpyAsync(&n_nl, temp + scan_temp_elems(nb) - 1, sizeof n_nl,
+                          hipMemcpyDeviceToHost, s));
+    TG_HIP(hipStreamSynchronize(s));
     if (n_nl >= (int64_t(1) << 31) - 2)
         throw std::runtime_error("GraphLoader: more than 2^31 lines in '" + c.name + "'");
-    exclusive_scan_i32(counts, offs, nb, temp, s);
     const int64_t n_seg = n_nl + 1;
     Carver p2(nullptr, 0);
     p2.take<int64_t>(n_seg);
@@ -510,10 +660,8 @@ void index_lines(tg_csv_s& c, hipStream_t s) {
     TG_LAUNCH_CHECK();
     header_kernel<<<1, 1, 0, s>>>(c.text, c.lb, c.le, pos + n_seg, c.meta.as<CsvMeta>());
     TG_LAUNCH_CHECK();
-    int32_t n_lines = 0;
-    TG_HIP(hipMemcpyAsync(&n_lines, pos + n_seg, sizeof n_lines, hipMemcpyDeviceToHost, s));
     const CsvMeta m = read_meta(c, s);  // synchronises
-    c.n_lines = n_lines;
+    c.n_lines = m.n_lines;
     c.header = m.header;
 }
 
@@ -596,14 +744,12 @@ void feature_shape(tg_csv_s& c, hipStream_t s) {
     c.cnt = c.node + n_data;
     c.tok = c.cnt + n_data;
     reset_meta(c, s);
-    feat_a_kernel<<<static_cast<unsigned>(n_data), kWave, 0, s>>>(
-        c.text, c.lb, c.le, c.header, c.node, c.cnt, c.meta.as<CsvMeta>());
+    feat_a_kernel<<<line_groups(n_data, 256), 256, 0, s>>>(c.text, c.lb, c.le, c.header, n_data,
+                                                           c.node, c.meta.as<CsvMeta>());
     TG_LAUNCH_CHECK();
-    int32_t first_cnt = 0;
-    TG_HIP(hipMemcpyAsync(&first_cnt, c.cnt, sizeof first_cnt, hipMemcpyDeviceToHost, s));
     const CsvMeta m = read_meta(c, s);
     c.rows = int64_t(m.max_id) + 1;
-    c.cols = std::max<int32_t>(first_cnt, 0);
+    c.cols = std::max<int32_t>(m.first_cnt, 0);
     c.shape_done = true;
 }
 
@@ -670,8 +816,8 @@ int tg_csv_parse_edges(tg_csv_t csv, int32_t* src, int32_t* dst, int64_t* max_id
         require(n_data == 0 || (src && dst), "GraphLoader::parse_edges: null output");
         tg::reset_meta(*csv, s);
         if (n_data > 0) {
-            tg::edges_kernel<<<tg::grid_of(n_data, 256), 256, 0, s>>>(
-                csv->text, csv->lb, csv->le, csv->header, n_data, src, dst,
+            tg::edges_kernel<<<tg::line_groups(n_data, 256), 256, 0, s>>>(
+                csv->text, csv->n_bytes, csv->lb, csv->le, csv->header, n_data, src, dst,
                 csv->meta.as<CsvMeta>());
             TG_LAUNCH_CHECK();
         }
@@ -731,8 +877,10 @@ int tg_csv_parse_features(tg_csv_t csv, float* out, int64_t n_rows, int64_t ld,
             TG_LAUNCH_CHECK();
         }
         tg::reset_meta(*csv, s);
-        tg::feat_b_kernel<<<static_cast<unsigned>(n_data), tg::kWave, 0, s>>>(
-            csv->text, csv->lb, csv->le, csv->header, csv->node, csv->cnt, winner.as<int32_t>(),
+        tg::feat_b_kernel<<<tg::line_groups(n_data, tg::kFeatWaves),
+                            tg::kFeatWaves * tg::kWave, 0, s>>>(
+            csv->text, csv->lb, csv->le, csv->header, n_data, csv->node, csv->cnt,
+            static_cast<int32_t>(cols), winner.as<int32_t>(),
             csv->pow10.as<tg::numparse::Pow10Entry>(), ld, out, csv->tok,
             csv->meta.as<CsvMeta>());
         TG_LAUNCH_CHECK();
