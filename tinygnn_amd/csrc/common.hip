@@ -2,8 +2,10 @@
 #include "common.hpp"
 #include "device_utils.hpp"
 
+#include <cstddef>
 #include <mutex>
 #include <string>
+#include <vector>
 
 namespace tg {
 
@@ -43,31 +45,36 @@ void DeviceBuffer::reset() {
 
 namespace {
 
-constexpr uint64_t kPoolKeep = uint64_t(512) << 20;
+constexpr size_t kKeepBytes = size_t(512) << 20;
+constexpr int kMaxDevices = 64;
 
-// The current device's pool, or null where it cannot be made.
-hipMemPool_t device_pool() {
-    constexpr int kMaxDevices = 64;
-    static std::mutex mu;
-    static hipMemPool_t pools[kMaxDevices] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-    std::lock_guard<std::mutex> lock(mu);
-    if (pools[dev] == nullptr) {
-        hipMemPoolProps props{};
-        props.allocType = hipMemAllocationTypePinned;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        hipMemPool_t pool = nullptr;
-        if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
-        uint64_t keep = kPoolKeep;
-        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
-            (void)hipMemPoolDestroy(pool);
-            return nullptr;
-        }
-        pools[dev] = pool;
-    }
-    return pools[dev];
+struct Block {
+    void* p;
+    size_t bytes;
+    hipEvent_t event;  // of the stream that freed it
+    bool idle;         // freed with the device idle: no event to wait for
+};
+
+struct Blocks {
+    std::mutex mu;
+    std::vector<Block> list;  // oldest first
+    size_t bytes = 0;
+};
+
+Blocks& blocks_of(int device) {
+    static Blocks* all = new Blocks[kMaxDevices];  // never destroyed: the runtime may go first
+    return all[device];
+}
+
+void give_back(const Block& b) {
+    (void)hipFree(b.p);  // waits for the device
+    (void)hipEventDestroy(b.event);
+}
+
+// Sizes of a call vary a little from one to the next: whole 64 KB, or 2 MB.
+size_t block_size(size_t bytes) {
+    const size_t unit = bytes <= (size_t(1) << 20) ? size_t(64) << 10 : size_t(2) << 20;
+    return (bytes + unit - 1) / unit * unit;
 }
 
 }  // namespace
@@ -76,48 +83,107 @@ void TempBuffer::allocate(size_t bytes, hipStream_t s) {
     reset();
     if (bytes == 0) return;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    hipMemPool_t pool = nullptr;
-    if (hipStreamIsCapturing(s, &capture) == hipSuccess &&
-        capture == hipStreamCaptureStatusNone)
-        pool = device_pool();
-    if (pool != nullptr) {
-        hipError_t e = hipMallocFromPoolAsync(&p_, bytes, pool, s);
-        if (e != hipSuccess) {  // give the pool's free memory back, then once more
-            (void)hipGetLastError();
-            (void)hipStreamSynchronize(s);
-            (void)hipMemPoolTrimTo(pool, 0);
-            e = hipMallocFromPoolAsync(&p_, bytes, pool, s);
+    const bool keep = hipStreamIsCapturing(s, &capture) == hipSuccess &&
+                      capture == hipStreamCaptureStatusNone &&
+                      hipGetDevice(&device_) == hipSuccess && device_ >= 0 &&
+                      device_ < kMaxDevices;
+    if (!keep) (void)hipGetLastError();
+    const size_t want = keep ? block_size(bytes) : bytes;
+    if (keep) {
+        Blocks& bl = blocks_of(device_);
+        Block b{};
+        {
+            std::lock_guard<std::mutex> lock(bl.mu);
+            size_t best = bl.list.size();
+            for (size_t i = 0; i < bl.list.size(); ++i)
+                if (bl.list[i].bytes >= want && bl.list[i].bytes / 2 <= want &&
+                    (best == bl.list.size() || bl.list[i].bytes < bl.list[best].bytes))
+                    best = i;
+            if (best < bl.list.size()) {
+                b = bl.list[best];
+                bl.list.erase(bl.list.begin() + static_cast<std::ptrdiff_t>(best));
+                bl.bytes -= b.bytes;
+            }
         }
-        if (e == hipSuccess) {
+        if (b.p != nullptr) {
+            hipError_t e = hipSuccess;
+            if (!b.idle && hipEventQuery(b.event) != hipSuccess) {
+                (void)hipGetLastError();  // not ready
+                e = hipStreamWaitEvent(s, b.event, 0);
+            }
+            if (e != hipSuccess) {
+                give_back(b);
+                TG_HIP(e);
+            }
+            p_ = b.p;
             n_ = bytes;
+            block_ = b.bytes;
+            event_ = b.event;
             stream_ = s;
-            pooled_ = true;
             return;
         }
-        p_ = nullptr;
+        const hipError_t e = hipEventCreateWithFlags(&event_, hipEventDisableTiming);
+        if (e != hipSuccess) {
+            event_ = nullptr;
+            TG_HIP(e);
+        }
     }
-    (void)hipGetLastError();
-    const hipError_t e = hipMalloc(&p_, bytes);
+    hipError_t e = hipMalloc(&p_, want);
+    if (e != hipSuccess && keep) {  // give the kept blocks back, then once more
+        (void)hipGetLastError();
+        std::vector<Block> old;
+        {
+            Blocks& bl = blocks_of(device_);
+            std::lock_guard<std::mutex> lock(bl.mu);
+            old.swap(bl.list);
+            bl.bytes = 0;
+        }
+        for (const Block& b : old) give_back(b);
+        e = hipMalloc(&p_, want);
+    }
     if (e != hipSuccess) {
         p_ = nullptr;
+        if (event_) (void)hipEventDestroy(event_);
+        event_ = nullptr;
         (void)hipGetLastError();
         throw AllocError("hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
                          hipGetErrorString(e));
     }
     n_ = bytes;
+    block_ = keep ? want : 0;
+    stream_ = s;
 }
 
 void TempBuffer::reset() {
     if (p_) {
-        if (pooled_)
-            (void)hipFreeAsync(p_, stream_);
-        else
-            (void)hipFree(p_);
+        const bool ordered =
+            block_ > 0 && block_ <= kKeepBytes &&
+            (idle_free_ || hipEventRecord(event_, stream_) == hipSuccess);
+        if (ordered) {
+            std::vector<Block> old;
+            {
+                Blocks& bl = blocks_of(device_);
+                std::lock_guard<std::mutex> lock(bl.mu);
+                bl.list.push_back(Block{p_, block_, event_, idle_free_});
+                bl.bytes += block_;
+                while (bl.bytes > kKeepBytes) {
+                    old.push_back(bl.list.front());
+                    bl.bytes -= bl.list.front().bytes;
+                    bl.list.erase(bl.list.begin());
+                }
+            }
+            for (const Block& b : old) give_back(b);
+        } else {
+            (void)hipGetLastError();
+            (void)hipFree(p_);  // waits for the device
+            if (event_) (void)hipEventDestroy(event_);
+        }
     }
     p_ = nullptr;
-    n_ = 0;
+    n_ = block_ = 0;
     stream_ = nullptr;
-    pooled_ = false;
+    event_ = nullptr;
+    idle_free_ = false;
 }
 
 void PinnedBuffer::reserve(size_t bytes) {

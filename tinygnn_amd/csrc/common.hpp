@@ -123,14 +123,16 @@ private:
     size_t n_ = 0;
 };
 
-// RAII device memory for a call's own temporaries, allocated and freed in
-// stream order from the library's pool of the current device: a call neither
-// waits for the GPU nor enters the driver once the pool is warm (hipMalloc and
-// hipFree of a 100 MB workspace on every call cost a SAGE-Max layer of 100K
-// nodes 5.3 of its 5.8 ms).  The pool keeps at most kPoolKeep freed bytes; the
-// rest goes back to the device at the next synchronisation, and all of it
-// before an allocation fails.  Where s is being captured the memory comes from
-// hipMalloc, which capture refuses.
+// RAII device memory for a call's own temporaries, in stream order: freed
+// blocks are kept (per device, at most kKeepBytes, oldest given back first, all
+// of them before an allocation fails) with an event of the freeing stream, which
+// the next user's stream waits for where it is not past yet.  So a warm call
+// neither waits for the GPU nor enters the driver: hipMalloc and hipFree of a
+// 100 MB workspace on every call cost a SAGE-Max layer of 100K nodes 5.3 of its
+// 5.8 ms.  (A hipMemPool's hipFreeAsync took 8 to 20 us of host time each, and
+// after some hundred loads of a 5M-edge graph the pool went to the driver on
+// every one: 1.7 ms a load, then 4.7.)  Where s is being captured the memory
+// comes from hipMalloc, which capture refuses.
 class TempBuffer {
 public:
     TempBuffer() = default;
@@ -140,20 +142,21 @@ public:
     TempBuffer& operator=(const TempBuffer&) = delete;
     void allocate(size_t bytes, hipStream_t s);  // discards contents
     void reset();
-    // Frees on the null stream instead of s, for memory that outlives the call
-    // (s may be gone); the device must be idle by then.
-    void outlive_stream() { stream_ = nullptr; }
+    // For memory that outlives the call (s may be gone by its end): the device
+    // must be idle when it is freed.
+    void outlive_stream() { idle_free_ = true; }
     void* get() const { return p_; }
     template <typename T> T* as() const { return static_cast<T*>(p_); }
     size_t size() const { return n_; }
-    // false: hipMalloc memory; freeing it waits for the device
-    bool pooled() const { return pooled_; }
 
 private:
     void* p_ = nullptr;
-    size_t n_ = 0;
+    size_t n_ = 0;       // bytes asked for
+    size_t block_ = 0;   // bytes of the kept block, 0: plain hipMalloc memory
+    int device_ = 0;
     hipStream_t stream_ = nullptr;
-    bool pooled_ = false;
+    hipEvent_t event_ = nullptr;
+    bool idle_free_ = false;
 };
 
 // RAII pinned host allocation (hipHostMalloc): small device-to-host results
