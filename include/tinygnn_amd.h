@@ -211,8 +211,8 @@ int tg_spmm_noalloc(int64_t m, int64_t k, int64_t f, int64_t nnz, const int32_t*
  * ops.hpp:76): C[m x n] = A[m x k] * B[k x n], with an optional fused
  * epilogue (bias add, then activation) that equals calling add_bias
  * (ops.cpp:622) and relu_inplace / elu_inplace afterwards.
- * algo: TG_GEMM_AUTO picks fp32 MFMA when n >= 64, k >= 32 and
- * m*n*k >= 2^32, else the in-order kernel; TG_GEMM_INORDER is bit-identical
+ * algo: TG_GEMM_AUTO may regroup the sums of large products (n >= 64, k >= 32
+ * and m*n*k >= 2^32; n < 64, k >= 32 and m*k >= 2^25), else in order; TG_GEMM_INORDER is bit-identical
  * to the reference (one fma chain over k ascending from 0 per output);
  * TG_GEMM_MFMA uses v_mfma_f32_16x16x4f32 (regrouped sums: within
  * tolerance, not bit-identical).

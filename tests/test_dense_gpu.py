@@ -36,6 +36,28 @@ def test_matmul_inorder_bitexact(gpu, restate, m, k, n):
     np.testing.assert_array_equal(bits(got), bits(restate.matmul(a, b)))
 
 
+@pytest.mark.parametrize("m,n", [(33, 1), (17, 16), (40000, 15),      # 16-row, 128-row tiles
+                                 (31, 17), (8200, 32),                # 32 columns: 16, 64 rows
+                                 (47, 33), (1, 130), (8300, 65)])     # 64 columns: 16, 64 rows
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 129, 200])
+def test_matmul_chain_tiles(gpu, restate, m, n, k):
+    """The in-order product's tiles at their edges: rows and columns past the
+    operands, a single partial tile of k, a last tile that overlaps the one
+    before, sums that underflow to -0 and infinities, bit for bit."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(m + 7 * n + 31 * k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    a[0] *= np.float32(1e-30)
+    b[:, 0] *= np.float32(1e-20)   # row 0, column 0: products round to +-0
+    a[m // 2, 0] = np.inf
+    got = tg.matmul(_t(gpu, a), _t(gpu, b), algo=tg.GEMM_INORDER).cpu().numpy()
+    want = restate.matmul(a, b)
+    nan = np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
 @pytest.mark.parametrize("m,k,n", [(128, 16, 128), (1000, 602, 256), (777, 256, 41),
                                    (300, 33, 130), (64, 1433, 64),
                                    # thin products (n <= 64: 16-column MFMA tiles), k not a

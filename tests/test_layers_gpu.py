@@ -53,6 +53,25 @@ def test_sage_concat_bitexact(gpu, restate, agg, f_in, f_out):
     np.testing.assert_array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("f_in", [3, 15, 16, 31, 33, 64, 65])
+@pytest.mark.parametrize("n,f_out", [(33, 7), (50, 9), (8300, 23), (40000, 8), (6000, 133)])
+def test_sage_dual_tiles_bitexact(gpu, restate, n, f_out, f_in):
+    """The in-order dual product's tiles (two k slots per k) and its tail
+    columns (from f_out rounded down to 8) at their edges, bit for bit."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(n + f_in * 10 + f_out)
+    a = random_csr(rng, n, n, avg_deg=2, max_deg=9, empty_frac=0.1)
+    h = rng.standard_normal((n, f_in)).astype(np.float32)
+    wn = rng.standard_normal((f_in, f_out)).astype(np.float32)
+    ws = rng.standard_normal((f_in, f_out)).astype(np.float32)
+    b = rng.standard_normal((1, f_out)).astype(np.float32)
+    want = restate.sage_layer(a, h, wn, ws, b, act=1, agg=1)
+    da = _dev(a)
+    got = tg.sage_forward(_plan(da, max(f_in, f_out)), da, _t(gpu, h), _t(gpu, wn), _t(gpu, ws),
+                          _t(gpu, b), act=1, agg=1, dataflow=tg.SAGE_CONCAT).cpu().numpy()
+    np.testing.assert_array_equal(bits(got), bits(want))
+
+
 @pytest.mark.parametrize("agg", [0, 1])
 def test_sage_aggregate_split_rows(gpu, restate, agg):
     import tinygnn_amd as tg

@@ -4,12 +4,11 @@
 // epilogues (ops.cpp:328-661): relu, leaky_relu, elu, sigmoid, tanh, gelu,
 // softmax, log_softmax, add_bias, plus edge_softmax (src/layers.cpp:768-822).
 //
-// Two GEMMs:
-//   * in order: one fma chain per output over k ascending from 0, through
-//     LDS tiles -- bit-identical to the reference; used for thin outputs
-//     (F_out 7/16/41) where the product is not a real contraction;
-//   * MFMA: v_mfma_f32_16x16x4f32, 128x128 workgroup tiles of four 64x64
-//     wavefront tiles, for the wide transforms (602->256, 4 heads x 64).
+// Two GEMMs, both on v_mfma_f32_16x16x4f32:
+//   * in order: one fma chain per output over k ascending from 0 --
+//     bit-identical to the reference; workgroup tiles of 16 to 128 rows;
+//   * MFMA: 128x128 workgroup tiles of four 64x64 wavefront tiles, the k
+//     order regrouped, for the wide transforms (602->256, 4 heads x 64).
 // Both fuse the bias add and the activation into the store.
 #include "common.hpp"
 #include "dense.hpp"
@@ -123,165 +122,266 @@ __device__ __forceinline__ void store_tiles_any(const GemmArgs& g, const v4f (&a
 }
 
 // ---------------------------------------------------------------------------
-// In-order GEMM (bit-exact)
+// In-order GEMM on the matrix cores (bit-exact).
+//
+// v_mfma_f32_16x16x4f32 computes each output as four fmas over its k slots
+// ascending, rounded after each and with denormals kept: compared with the
+// chain fma(a3, b3, fma(a2, b2, fma(a1, b1, fma(a0, b0, c)))) on the CPU
+// over normal, denormal, overflowing, infinite and NaN operands, every bit
+// of 460,000 outputs agreed.  So with lane group q of a step feeding k =
+// 4 s + q, an output is the reference's one fma chain over k ascending from
+// 0.  The dual product's chain takes the pairs in turn, so its operands are
+// interleaved per k in LDS and the same steps run over 2 k slots.
+//
+// A workgroup computes 16 MI WR x 16 NJ WC outputs (WR x WC wavefronts of
+// MI x NJ MFMA tiles; of four wavefronts the others only load).  Tiles of KT
+// k slots go through two LDS buffers, two further tiles in flight in
+// registers: a small product has one or two workgroups per CU and a chain of
+// K / 4 dependent MFMAs of 32 cycles (K = 1433: 5 us), and what held it was
+// the wait for each tile.  A lies [row][k] at a pitch of KT + 4 floats and B
+// [k][column] at a pitch of 16 (mod 64), so both operands' 32-bit reads (16
+// rows x 4 k; 4 k x 16 columns) fall in 64 distinct banks.
+//
+// FULL: at least one tile of k.  The last tile then ends at K, so every load
+// is whole and unguarded, and the slots of it that the tile before held are
+// made neutral: A = -0, B = +0, whose product -0 leaves any accumulator,
+// -0 included, as it is.  Not FULL: one partial tile, loads clamped into the
+// operands, the slots from K on neutral.  Rows past M and columns past N
+// read the last one; their outputs are not stored.
+//
+// Against the one-fma-per-lane kernels that this replaces, same bits, us:
+// 2,708 x 1,433 x 16 30.4 -> 15.9, x 64 57.7 -> 21.6, 20,000 x 500 x 16 34 ->
+// 12.5, 300,000 x 100 x 30 80 -> 45, 232,965 x 16 x 41 44 -> 27, 100,003 x
+// 257 x 121 130 -> 91 (68 TFLOP/s), 100,000 x 128 x 256 131 -> 87; SAGE's
+// layer around the dual 2,708 x 1,433 x 64 129 -> 76, 100,000 x 64 x 40 149
+// -> 56.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int TM, int TN, bool DUAL>
-__global__ __launch_bounds__(256) void gemm_inorder_kernel(GemmArgs g) {
-    constexpr int BK = 16;
-    constexpr int TX = BN / TN;
-    constexpr int TY = BM / TM;
-    static_assert(TX * TY == 256, "256 threads");
+template <int MI, int NJ, int WR, int WC, int KT, bool DUAL, bool FULL>
+__global__ __launch_bounds__(256) void gemm_chain_kernel(GemmArgs g) {
+    constexpr int BM = 16 * MI * WR, BN = 16 * NJ * WC;
+    constexpr int PA = KT + 4, PB = BN % 32 == 16 ? BN : BN + 16;
     constexpr int NP = DUAL ? 2 : 1;
-    __shared__ float As[NP][BK][BM];
-    __shared__ float Bs[NP][BK][BN];
-    const int tx = threadIdx.x % TX;
-    const int ty = threadIdx.x / TX;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * BM;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.y) * BN;
+    constexpr int KR = KT / NP;             // k of a tile
+    constexpr int CPR = KR / 4;             // A chunks of 4 k per row and pair
+    constexpr int NA = BM * CPR;            // ... of a tile; below 256, threads load them twice
+    constexpr int LA = (NA + 255) / 256;    // ... per thread
+    constexpr int LB = KT * BN / 256;       // B values per thread
+    constexpr int SB = 256 / BN;            // B slots between a thread's values
+    static_assert((NA % 256 == 0 || 256 % NA == 0) && KT * BN % 256 == 0 && SB % NP == 0, "tile");
+    __shared__ __attribute__((aligned(16))) float As[2][BM][PA];
+    __shared__ __attribute__((aligned(16))) float Bs[2][KT][PB];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int wm = (wave / WC) * 16 * MI, wn = (wave % WC) * 16 * NJ;
+    const bool works = wave < WR * WC;
     const int64_t M = g.m, N = g.n, K = g.k1;
+    // a row tile's column tiles follow one another on one XCD (its L2 then
+    // holds that A), as in gemm_mfma_kernel
+    const int64_t mt = (M + BM - 1) / BM, ntl = (N + BN - 1) / BN;
+    const int64_t xj = blockIdx.x / 8;
+    const int64_t mtile = (xj / ntl) * 8 + blockIdx.x % 8;
+    if (mtile >= mt) return;  // before any barrier: the whole workgroup
+    const int64_t m0 = mtile * BM, n0 = (xj % ntl) * BN;
+    const int64_t nt = (K + KR - 1) / KR;
 
-    float acc[TM][TN];
+    const float* pa[NP][LA];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = 0.0f;
+    for (int t = 0; t < LA; ++t) {
+        const int e = (tid + 256 * t) % NA;
+        const int64_t gm = m0 + e / CPR < M ? m0 + e / CPR : M - 1;
+        pa[0][t] = g.a1 + gm * g.lda1;
+        if constexpr (DUAL) pa[1][t] = g.a2 + gm * g.lda2;
+    }
+    const int bslot = tid / BN;  // this thread's first B slot; its parity is its pair
+    const bool second = DUAL && (bslot & 1);
+    const int64_t ldb = second ? g.ldb2 : g.ldb1;
+    const int64_t gn = n0 + tid % BN < N ? n0 + tid % BN : N - 1;
+    const float* pb = (second ? g.b2 : g.b1) + gn;
+    const int kb = bslot / NP;
 
-    // tail columns (dual only): tail_from is a multiple of 8, so a thread's
-    // TN consecutive columns are all tail or all not
-    const bool tail = DUAL && g.tail_from >= 0 && (n0 + tx * TN) >= g.tail_from;
-
-    for (int64_t k0 = 0; k0 < K; k0 += BK) {
+    struct Regs {
+        v4f a[NP][LA];
+        float b[LB];
+    };
+    auto fetch = [&](int64_t kt, Regs& x) {
+        if constexpr (FULL) {
+            const int64_t k0 = kt * KR < K - KR ? kt * KR : K - KR;
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const float* A = p ? g.a2 : g.a1;
-            const float* B = p ? g.b2 : g.b1;
-            const int64_t lda = p ? g.lda2 : g.lda1;
-            const int64_t ldb = p ? g.ldb2 : g.ldb1;
-            for (int e = threadIdx.x; e < BM * BK; e += 256) {
-                const int mm = e / BK, kk = e % BK;
-                const int64_t gm = m0 + mm, gk = k0 + kk;
-                As[p][kk][mm] = (gm < M && gk < K) ? A[gm * lda + gk] : 0.0f;
-            }
-            for (int e = threadIdx.x; e < BN * BK; e += 256) {
-                const int kk = e / BN, nn = e % BN;
-                const int64_t gk = k0 + kk, gn = n0 + nn;
-                Bs[p][kk][nn] = (gk < K && gn < N) ? B[gk * ldb + gn] : 0.0f;
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int t = 0; t < LA; ++t)
+                    x.a[p][t] = *reinterpret_cast<const Float4Dw*>(pa[p][t] + k0 +
+                                                                   4 * ((tid + 256 * t) % CPR));
+            const float* b = pb + (k0 + kb) * ldb;
+#pragma unroll
+            for (int t = 0; t < LB; ++t) x.b[t] = b[t * (SB / NP) * ldb];
+        } else {
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int t = 0; t < LA; ++t)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int64_t k = 4 * ((tid + 256 * t) % CPR) + u;
+                        x.a[p][t][u] = pa[p][t][k < K ? k : K - 1];
+                    }
+#pragma unroll
+            for (int t = 0; t < LB; ++t) {
+                const int64_t k = kb + t * (SB / NP);
+                x.b[t] = pb[(k < K ? k : K - 1) * ldb];
             }
         }
-        __syncthreads();
-        const int kmax = static_cast<int>(K - k0 < BK ? K - k0 : BK);
-        for (int kk = 0; kk < kmax; ++kk) {
-            float a[TM], b[TN];
+    };
+    auto stage = [&](int64_t kt, int buf, Regs& x) {
+        // k of the tile that are its own: [lo, hi)
+        const int lo = FULL && kt * KR > K - KR ? static_cast<int>(kt * KR - (K - KR)) : 0;
+        const int hi = FULL ? KR : static_cast<int>(K);
+        if (lo > 0 || hi < KR) {  // uniform
 #pragma unroll
-            for (int i = 0; i < TM; ++i) a[i] = As[0][kk][ty * TM + i];
+            for (int t = 0; t < LA; ++t)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) b[j] = Bs[0][kk][tx * TN + j];
-            if constexpr (DUAL) {
-                float a2[TM], b2[TN];
+                for (int u = 0; u < 4; ++u) {
+                    const int k = 4 * ((tid + 256 * t) % CPR) + u;
 #pragma unroll
-                for (int i = 0; i < TM; ++i) a2[i] = As[NP - 1][kk][ty * TM + i];
-#pragma unroll
-                for (int j = 0; j < TN; ++j) b2[j] = Bs[NP - 1][kk][tx * TN + j];
-                if (tail) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j)
-                            acc[i][j] = acc[i][j] + __builtin_fmaf(a[i], b[j], a2[i] * b2[j]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            const float t = __builtin_fmaf(a[i], b[j], acc[i][j]);
-                            acc[i][j] = __builtin_fmaf(a2[i], b2[j], t);
-                        }
+                    for (int p = 0; p < NP; ++p)
+                        x.a[p][t][u] = k >= lo && k < hi ? x.a[p][t][u] : -0.0f;
                 }
-            } else {
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+            for (int t = 0; t < LB; ++t) {
+                const int k = kb + t * (SB / NP);
+                x.b[t] = k >= lo && k < hi ? x.b[t] : 0.0f;
             }
         }
+#pragma unroll
+        for (int t = 0; t < LA; ++t) {
+            const int e = (tid + 256 * t) % NA;
+            float* at = &As[buf][e / CPR][4 * NP * (e % CPR)];
+            if constexpr (DUAL) {
+                const v4f a = x.a[0][t], b = x.a[1][t];
+                *reinterpret_cast<v4f*>(at) = v4f{a[0], b[0], a[1], b[1]};
+                *reinterpret_cast<v4f*>(at + 4) = v4f{a[2], b[2], a[3], b[3]};
+            } else {
+                *reinterpret_cast<v4f*>(at) = x.a[0][t];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < LB; ++t) Bs[buf][bslot + t * SB][tid % BN] = x.b[t];
+    };
+
+    v4f acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](int buf) {
+        if (!works) return;
+        constexpr int U = MI * NJ == 1 ? 16 : 4;  // steps whose operands are read ahead
+#pragma unroll 1
+        for (int s0 = 0; s0 < KT / 4; s0 += U) {
+            static_assert(KT / 4 % U == 0, "steps");
+            float a[U][MI], b[U][NJ];
+#pragma unroll
+            for (int s = 0; s < U; ++s) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) a[s][i] = As[buf][wm + i * 16 + r][4 * (s0 + s) + q];
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) b[s][j] = Bs[buf][4 * (s0 + s) + q][wn + j * 16 + r];
+            }
+#pragma unroll
+            for (int s = 0; s < U; ++s)
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][i], b[s][j],
+                                                                         acc[i][j], 0, 0, 0);
+        }
+    };
+
+    if (nt == 1) {
+        Regs x;
+        fetch(0, x);
+        stage(0, 0, x);
         __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int64_t gm = m0 + ty * TM + i;
-        if (gm >= M) continue;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int64_t gn = n0 + tx * TN + j;
-            if (gn < N) g.c[c_index(g, gm, gn)] = epi_out(g, acc[i][j], gm, gn);
+        compute(0);
+    } else if (FULL && nt > 1) {
+        // Fetches past the last tile load it again: no branch, so no wait
+        // for loads that a branch might have issued.
+        Regs x0, x1;
+        fetch(0, x0);
+        fetch(1, x1);
+        stage(0, 0, x0);
+        fetch(2, x0);
+        __syncthreads();
+        for (int64_t kt = 0; kt < nt; kt += 2) {
+            if (kt + 1 < nt) stage(kt + 1, 1, x1);
+            fetch(kt + 3, x1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(0);
+            __syncthreads();
+            if (kt + 1 >= nt) break;
+            if (kt + 2 < nt) stage(kt + 2, 0, x0);
+            fetch(kt + 4, x0);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(1);
+            __syncthreads();
         }
     }
+    if (works) store_tiles_any(g, acc, m0 + wm, n0 + wn, q, r);
 }
 
 // ---------------------------------------------------------------------------
-// In-order GEMM for small products (bit-exact; m n <= 2^21, e.g. the
-// Cora-scale transforms): one output per thread, a workgroup covers BM x BN
-// outputs (BM = 256 / BN), so a 2,708-row product gets 170-680 workgroups
-// instead of 11-22, and the k loop runs over 64-wide tiles with the next
-// tile loaded into registers while the current one is consumed from LDS.
-// Each output is one fma chain over k ascending from 0 (padded k is never
-// accumulated); DUAL interleaves the pairs per k and applies the scalar tail
-// exactly as gemm_inorder_kernel.
+// The dual product's scalar-tail columns (bit-exact): at most 8 columns, each
+// output c = c + fma(a1, b1, a2 * b2) over k ascending, one per thread.  The
+// fmas of successive k do not depend on each other, only the adds do, so
+// what bounds it is the operands' way through LDS: both lie with k
+// innermost and come as 128-bit reads (2,708 x 1,433 x 1 of a SAGE layer with
+// 41 outputs: 80 us with 32-bit reads, 32 now; rows and columns at a 68-float pitch:
+// the 8 of each that a wavefront reads fall in distinct banks), the next
+// tile in registers meanwhile.  k past K is neutral: A = -0, B = +0 adds -0.
 // ---------------------------------------------------------------------------
-constexpr int kSBK = 64;
+constexpr int kDTRows = 32, kDTCols = 8, kDTK = 64, kDTP = kDTK + 4;
 
-template <int BN, bool DUAL>
-__global__ __launch_bounds__(256) void gemm_inorder_small_kernel(GemmArgs g) {
-    constexpr int BM = 256 / BN;
-    constexpr int NP = DUAL ? 2 : 1;
-    constexpr int LA = BM * kSBK / 256;  // A values per thread per tile
-    constexpr int LB = kSBK * BN / 256;  // B values per thread per tile
-    static_assert(LA >= 1 && LB >= 1, "tile shape");
-    __shared__ float As[2][NP][kSBK][BM];
-    __shared__ float Bs[2][NP][kSBK][BN];
-    const int tx = threadIdx.x % BN, ty = threadIdx.x / BN;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * BM;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.y) * BN;
+__global__ __launch_bounds__(256) void gemm_dual_tail_kernel(GemmArgs g) {
+    __shared__ __attribute__((aligned(16))) float As[2][2][kDTRows][kDTP];
+    __shared__ __attribute__((aligned(16))) float Bs[2][2][kDTCols][kDTP];
+    constexpr int LA = kDTRows * kDTK / 256, LB = kDTCols * kDTK / 256;
+    const int tid = threadIdx.x, tx = tid % kDTCols, ty = tid / kDTCols;
+    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * kDTRows;
     const int64_t M = g.m, N = g.n, K = g.k1;
-    const int64_t nt = (K + kSBK - 1) / kSBK;
-    const bool tail = DUAL && g.tail_from >= 0 && (n0 + tx) >= g.tail_from;
+    const int64_t nt = (K + kDTK - 1) / kDTK;
+    const int64_t bn = tx < N ? tx : N - 1;
 
-    float ra[NP][LA], rb[NP][LB];
+    float ra[2][LA], rb[2][LB];
     auto fetch = [&](int64_t kt) {
-        const int64_t k0 = kt * kSBK;
+        const int64_t k0 = kt * kDTK;
+        const int64_t ka = k0 + tid % kDTK;
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
+        for (int p = 0; p < 2; ++p) {
             const float* A = p ? g.a2 : g.a1;
             const float* B = p ? g.b2 : g.b1;
-            const int64_t lda = p ? g.lda2 : g.lda1;
-            const int64_t ldb = p ? g.ldb2 : g.ldb1;
+            const int64_t lda = p ? g.lda2 : g.lda1, ldb = p ? g.ldb2 : g.ldb1;
 #pragma unroll
             for (int t = 0; t < LA; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                const int64_t gm = m0 + e / kSBK, gk = k0 + e % kSBK;
-                ra[p][t] = (gm < M && gk < K) ? A[gm * lda + gk] : 0.0f;
+                const int64_t gm = m0 + tid / kDTK + t * (256 / kDTK);
+                ra[p][t] = ka < K ? A[(gm < M ? gm : M - 1) * lda + ka] : -0.0f;
             }
 #pragma unroll
             for (int t = 0; t < LB; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                const int64_t gk = k0 + e / BN, gn = n0 + e % BN;
-                rb[p][t] = (gk < K && gn < N) ? B[gk * ldb + gn] : 0.0f;
+                const int64_t kb = k0 + ty + t * (256 / kDTCols);
+                rb[p][t] = kb < K ? B[kb * ldb + bn] : 0.0f;
             }
         }
     };
     auto stage = [&](int buf) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
+        for (int p = 0; p < 2; ++p) {
 #pragma unroll
-            for (int t = 0; t < LA; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                As[buf][p][e % kSBK][e / kSBK] = ra[p][t];
-            }
+            for (int t = 0; t < LA; ++t)
+                As[buf][p][tid / kDTK + t * (256 / kDTK)][tid % kDTK] = ra[p][t];
 #pragma unroll
-            for (int t = 0; t < LB; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                Bs[buf][p][e / BN][e % BN] = rb[p][t];
-            }
+            for (int t = 0; t < LB; ++t) Bs[buf][p][tx][ty + t * (256 / kDTCols)] = rb[p][t];
         }
     };
 
@@ -294,287 +394,20 @@ __global__ __launch_bounds__(256) void gemm_inorder_small_kernel(GemmArgs g) {
     for (int64_t kt = 0; kt < nt; ++kt) {
         const int cb = static_cast<int>(kt & 1);
         if (kt + 1 < nt) fetch(kt + 1);
-        const int64_t k0 = kt * kSBK;
-        const int kmax = static_cast<int>(K - k0 < kSBK ? K - k0 : kSBK);
-        // the dual form is chosen outside the k loop (a branch inside it
-        // cost Cora-scale dual n x 1433 x 64 about a third of its time)
-        if (DUAL && tail) {
-            for (int kk = 0; kk < kmax; ++kk) {
-                const float a = As[cb][0][kk][ty], b = Bs[cb][0][kk][tx];
-                const float a2 = As[cb][NP - 1][kk][ty], b2 = Bs[cb][NP - 1][kk][tx];
-                acc = acc + __builtin_fmaf(a, b, a2 * b2);
-            }
-        } else {
-            for (int kk = 0; kk < kmax; ++kk) {
-                const float a = As[cb][0][kk][ty], b = Bs[cb][0][kk][tx];
-                if constexpr (DUAL) {
-                    const float a2 = As[cb][NP - 1][kk][ty], b2 = Bs[cb][NP - 1][kk][tx];
-                    acc = __builtin_fmaf(a2, b2, __builtin_fmaf(a, b, acc));
-                } else {
-                    acc = __builtin_fmaf(a, b, acc);
-                }
-            }
+        auto at = [&](const float* p, int k) { return *reinterpret_cast<const v4f*>(p + k); };
+#pragma unroll 4
+        for (int k = 0; k < kDTK; k += 4) {
+            const v4f a1 = at(As[cb][0][ty], k), a2 = at(As[cb][1][ty], k);
+            const v4f b1 = at(Bs[cb][0][tx], k), b2 = at(Bs[cb][1][tx], k);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                acc = acc + __builtin_fmaf(a1[u], b1[u], a2[u] * b2[u]);
         }
         if (kt + 1 < nt) stage(cb ^ 1);
         __syncthreads();
     }
-    const int64_t gm = m0 + ty, gn = n0 + tx;
-    if (gm < M && gn < N) g.c[c_index(g, gm, gn)] = epi_out(g, acc, gm, gn);
-}
-
-// ---------------------------------------------------------------------------
-// In-order GEMM for small products in 64-column slabs (bit-exact; the
-// Cora-scale dual n x 1433 x 64 SAGE transform): a wavefront computes TM
-// rows x 64 columns, one column per lane.  The rows are wave-uniform, so
-// their A values come through scalar loads (s_load_dwordx16, no LDS); the
-// workgroup's four wavefronts share each k-tile of kRKT rows of B through
-// LDS (two buffers, the next tile loaded into registers while the current
-// one is consumed).  Every output is one fma chain over k ascending from
-// 0, never over padded k; DUAL interleaves the pairs per k and applies the
-// reference's scalar tail, as gemm_inorder_kernel.  A tile's A values (TM x
-// kRKT per pair) must fit the scalar registers.  Measured on the dual
-// 2708 x 1433 x 64 product (Cora-synth SAGE forward, 204 us with
-// gemm_inorder_small_kernel): TM 1 / kRKT 32 145 us, kRKT 16 154 us, kRKT
-// 64 200 us (scalar spills), TM 2 169 us, TM 4 255 us; the single product
-// (GAT) is no faster than gemm_inorder_small_kernel and stays there.
-// ---------------------------------------------------------------------------
-template <int TM, int kRKT, bool DUAL>
-__global__ __launch_bounds__(256) void gemm_inorder_rows_kernel(GemmArgs g) {
-    constexpr int NP = DUAL ? 2 : 1;
-    constexpr int LB = kRKT * 64 / 256;  // B values per thread per tile and pair
-    __shared__ float Bs[2][NP][kRKT][64];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int64_t M = g.m, N = g.n, K = g.k1;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.y) * 64;
-    const int64_t m0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * TM;
-    const int64_t nt = (K + kRKT - 1) / kRKT;
-    // the wave's rows of A (clamped for the loads; rows >= M are not stored)
-    const float* ar[NP][TM];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int r = 0; r < TM; ++r) {
-            const int64_t row = m0 + r < M ? m0 + r : M - 1;
-            ar[p][r] = p ? g.a2 + row * g.lda2 : g.a1 + row * g.lda1;
-        }
-    const bool tail = DUAL && g.tail_from >= 0 && (n0 + lane) >= g.tail_from;
-
-    float rb[NP][LB];
-    auto fetch = [&](int64_t kt) {
-        const int64_t k0 = kt * kRKT;
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const float* B = p ? g.b2 : g.b1;
-            const int64_t ldb = p ? g.ldb2 : g.ldb1;
-#pragma unroll
-            for (int t = 0; t < LB; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                const int64_t gk = k0 + e / 64, gn = n0 + e % 64;
-                rb[p][t] = (gk < K && gn < N) ? B[gk * ldb + gn] : 0.0f;
-            }
-        }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-#pragma unroll
-            for (int t = 0; t < LB; ++t) {
-                const int e = threadIdx.x + 256 * t;
-                Bs[buf][p][e / 64][e % 64] = rb[p][t];
-            }
-    };
-
-    float acc[TM];
-#pragma unroll
-    for (int r = 0; r < TM; ++r) acc[r] = 0.0f;
-    // one k step of every row: plain (tail = false) or the scalar tail form
-    auto step = [&](int cb, int64_t k, int kk, bool tl) {
-        const float b1 = Bs[cb][0][kk][lane];
-        const float b2 = Bs[cb][NP - 1][kk][lane];
-#pragma unroll
-        for (int r = 0; r < TM; ++r) {
-            const float a1 = ar[0][r][k];
-            if constexpr (DUAL) {
-                const float a2 = ar[NP - 1][r][k];
-                acc[r] = tl ? acc[r] + __builtin_fmaf(a1, b1, a2 * b2)
-                            : __builtin_fmaf(a2, b2, __builtin_fmaf(a1, b1, acc[r]));
-            } else {
-                acc[r] = __builtin_fmaf(a1, b1, acc[r]);
-            }
-        }
-    };
-    if (nt > 0) {
-        fetch(0);
-        stage(0);
-    }
-    __syncthreads();
-    for (int64_t kt = 0; kt < nt; ++kt) {
-        const int cb = static_cast<int>(kt & 1);
-        if (kt + 1 < nt) fetch(kt + 1);
-        const int64_t k0 = kt * kRKT;
-        const int kmax = static_cast<int>(K - k0 < kRKT ? K - k0 : kRKT);
-        // the dual form is chosen outside the k loop
-        if (kmax == kRKT) {
-            if (DUAL && tail) {
-#pragma unroll
-                for (int kk = 0; kk < kRKT; ++kk) step(cb, k0 + kk, kk, true);
-            } else {
-#pragma unroll
-                for (int kk = 0; kk < kRKT; ++kk) step(cb, k0 + kk, kk, false);
-            }
-        } else {
-            if (DUAL && tail) {
-                for (int kk = 0; kk < kmax; ++kk) step(cb, k0 + kk, kk, true);
-            } else {
-                for (int kk = 0; kk < kmax; ++kk) step(cb, k0 + kk, kk, false);
-            }
-        }
-        if (kt + 1 < nt) stage(cb ^ 1);
-        __syncthreads();
-    }
-    const int64_t gn = n0 + lane;
-#pragma unroll
-    for (int r = 0; r < TM; ++r) {
-        const int64_t gm = m0 + r;
-        if (gm < M && gn < N) g.c[c_index(g, gm, gn)] = epi_out(g, acc[r], gm, gn);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Wide in-order GEMM (bit-exact, n > 32): 128x128 workgroup tile, an 8x8
-// register micro-tile per thread, BK = 8, two LDS buffers with register
-// prefetch.  Each output is still one fma chain over k ascending from 0 (the
-// k loop is outermost, and no padded k is ever accumulated), so the result
-// equals the reference's (i,k,j) loop bit for bit; DUAL interleaves the two
-// products per k exactly as the in-order kernel above.
-// ---------------------------------------------------------------------------
-constexpr int kWBM = 128, kWBN = 128, kWBK = 8;
-
-template <int VA, bool DUAL>
-__global__ __launch_bounds__(256) void gemm_inorder_wide_kernel(GemmArgs g) {
-    constexpr int NP = DUAL ? 2 : 1;
-    __shared__ __attribute__((aligned(16))) float As[2][NP][kWBK][kWBM];
-    __shared__ __attribute__((aligned(16))) float Bs[2][NP][kWBK][kWBN];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x) * kWBM;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.y) * kWBN;
-    const int64_t M = g.m, N = g.n, K = g.k1;
-    const int64_t nt = (K + kWBK - 1) / kWBK;
-    // loads: A row ar, 4 k from ak; B row bk, 4 n from bn
-    const int ar = threadIdx.x >> 1, ak = (threadIdx.x & 1) * 4;
-    const int bk = threadIdx.x >> 5, bn = (threadIdx.x & 31) * 4;
-    float ra[NP][4], rb[NP][4];
-
-    auto fetch = [&](int64_t kt) {
-        const int64_t k0 = kt * kWBK;
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const float* A = p ? g.a2 : g.a1;
-            const float* B = p ? g.b2 : g.b1;
-            const int64_t lda = p ? g.lda2 : g.lda1;
-            const int64_t ldb = p ? g.ldb2 : g.ldb1;
-            const int64_t gm = m0 + ar, ka = k0 + ak;
-            const float* pa = A + (gm < M ? gm : 0) * lda + ka;
-            const int64_t va = gm < M ? K - ka : 0;
-            if (VA == 4 && va >= 4) {
-                const Float4Dw t = *reinterpret_cast<const Float4Dw*>(pa);
-                ra[p][0] = t.x; ra[p][1] = t.y; ra[p][2] = t.z; ra[p][3] = t.w;
-            } else {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) ra[p][u] = u < va ? pa[u] : 0.0f;
-            }
-            const int64_t kb = k0 + bk, nb = n0 + bn;
-            const float* pb = B + (kb < K ? kb : 0) * ldb + nb;
-            const int64_t vb = kb < K ? N - nb : 0;
-            if (vb >= 4) {
-                const Float4Dw t = *reinterpret_cast<const Float4Dw*>(pb);
-                rb[p][0] = t.x; rb[p][1] = t.y; rb[p][2] = t.z; rb[p][3] = t.w;
-            } else {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) rb[p][u] = u < vb ? pb[u] : 0.0f;
-            }
-        }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) As[buf][p][ak + u][ar] = ra[p][u];
-            *reinterpret_cast<float4*>(&Bs[buf][p][bk][bn]) =
-                make_float4(rb[p][0], rb[p][1], rb[p][2], rb[p][3]);
-        }
-    };
-
-    float acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0f;
-    // tail columns (dual only): tail_from is a multiple of 8, so a thread's
-    // eight consecutive columns are all tail or all not
-    const bool tail = DUAL && g.tail_from >= 0 && (n0 + tx * 8) >= g.tail_from;
-
-    if (nt > 0) {
-        fetch(0);
-        stage(0);
-    }
-    __syncthreads();
-    for (int64_t kt = 0; kt < nt; ++kt) {
-        const int cb = static_cast<int>(kt & 1);
-        if (kt + 1 < nt) fetch(kt + 1);
-        const int kmax = static_cast<int>(K - kt * kWBK < kWBK ? K - kt * kWBK : kWBK);
-        for (int kk = 0; kk < kmax; ++kk) {
-            float a[NP][8], b[NP][8];
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const float4 a0 = *reinterpret_cast<const float4*>(&As[cb][p][kk][ty * 8]);
-                const float4 a1 = *reinterpret_cast<const float4*>(&As[cb][p][kk][ty * 8 + 4]);
-                const float4 b0 = *reinterpret_cast<const float4*>(&Bs[cb][p][kk][tx * 8]);
-                const float4 b1 = *reinterpret_cast<const float4*>(&Bs[cb][p][kk][tx * 8 + 4]);
-                a[p][0] = a0.x; a[p][1] = a0.y; a[p][2] = a0.z; a[p][3] = a0.w;
-                a[p][4] = a1.x; a[p][5] = a1.y; a[p][6] = a1.z; a[p][7] = a1.w;
-                b[p][0] = b0.x; b[p][1] = b0.y; b[p][2] = b0.z; b[p][3] = b0.w;
-                b[p][4] = b1.x; b[p][5] = b1.y; b[p][6] = b1.z; b[p][7] = b1.w;
-            }
-            if constexpr (DUAL) {
-                if (tail) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            acc[i][j] = acc[i][j] +
-                                        __builtin_fmaf(a[0][i], b[0][j], a[NP - 1][i] * b[NP - 1][j]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            const float t = __builtin_fmaf(a[0][i], b[0][j], acc[i][j]);
-                            acc[i][j] = __builtin_fmaf(a[NP - 1][i], b[NP - 1][j], t);
-                        }
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        acc[i][j] = __builtin_fmaf(a[0][i], b[0][j], acc[i][j]);
-            }
-        }
-        if (kt + 1 < nt) stage(cb ^ 1);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int64_t gm = m0 + ty * 8 + i;
-        if (gm >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int64_t gn = n0 + tx * 8 + j;
-            if (gn < N) g.c[c_index(g, gm, gn)] = epi_out(g, acc[i][j], gm, gn);
-        }
-    }
+    const int64_t gm = m0 + ty;
+    if (gm < M && tx < N) g.c[c_index(g, gm, tx)] = epi_out(g, acc, gm, tx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1023,58 +856,68 @@ unsigned ew_grid(int64_t n) {
     return static_cast<unsigned>(b);
 }
 
-template <int BM, int BN, int TM, int TN, bool DUAL>
-void launch_inorder(const GemmArgs& g, hipStream_t s) {
-    dim3 grid(static_cast<unsigned>(ceil_div(g.m, BM)), static_cast<unsigned>(ceil_div(g.n, BN)));
-    gemm_inorder_kernel<BM, BN, TM, TN, DUAL><<<grid, 256, 0, s>>>(g);
+template <int MI, int NJ, int WR, int WC, int KT, bool DUAL, bool FULL>
+void launch_chain_as(const GemmArgs& g, hipStream_t s) {
+    const int64_t wgs =
+        8 * ceil_div(ceil_div(g.m, 16 * MI * WR), 8) * ceil_div(g.n, 16 * NJ * WC);
+    require(wgs < (int64_t(1) << 31), "matmul: too many row tiles");
+    gemm_chain_kernel<MI, NJ, WR, WC, KT, DUAL, FULL>
+        <<<static_cast<unsigned>(wgs), 256, 0, s>>>(g);
     TG_LAUNCH_CHECK();
 }
 
-template <int BN, bool DUAL>
-void launch_inorder_small(const GemmArgs& g, hipStream_t s) {
-    dim3 grid(static_cast<unsigned>(ceil_div(g.m, 256 / BN)),
-              static_cast<unsigned>(ceil_div(g.n, BN)));
-    gemm_inorder_small_kernel<BN, DUAL><<<grid, 256, 0, s>>>(g);
-    TG_LAUNCH_CHECK();
+template <int MI, int NJ, int WR, int WC, int KT, bool DUAL>
+void launch_chain_kt(const GemmArgs& g, hipStream_t s) {
+    if (g.k1 >= KT / (DUAL ? 2 : 1))
+        launch_chain_as<MI, NJ, WR, WC, KT, DUAL, true>(g, s);
+    else
+        launch_chain_as<MI, NJ, WR, WC, KT, DUAL, false>(g, s);
 }
 
-template <int TM, int KT, bool DUAL>
-void launch_inorder_rows(const GemmArgs& g, hipStream_t s) {
-    dim3 grid(static_cast<unsigned>(ceil_div(g.m, 4 * TM)), static_cast<unsigned>(ceil_div(g.n, 64)));
-    gemm_inorder_rows_kernel<TM, KT, DUAL><<<grid, 256, 0, s>>>(g);
-    TG_LAUNCH_CHECK();
-}
-
+// The in-order tile for a size.  Small products take 16-row tiles, for the
+// number of workgroups (a chain's length does not depend on the tile);
+// larger ones take tiles that read B less often.  Either side of each line,
+// us: n = 16: 20,000 x 500 12.5 / 16.4, 60,000 x 300 19.8 / 18.8; n <= 32:
+// 2,708 x 1,433 x 32 17.7 / 32.1, 30,000 x 700 x 24 32.4 / 26.4; n > 32:
+// 12,000 x 300 x 60 13.3 / 15.2, 20,000 x 300 x 60 22.0 / 21.1; k < 32, where
+// a 32-slot tile is mostly padding: 400,000 x 8 x 200 140 against 176.
 template <bool DUAL>
-void dispatch_inorder(const GemmArgs& g, hipStream_t s) {
-    // Small products (m n <= 2^21): one output per thread, many workgroups
-    // (Cora-scale GCN / SAGE / GAT forwards); the kernels below give such
-    // products a few dozen workgroups at most.
-    if (g.m * g.n <= (int64_t(1) << 21)) {
-        if (g.n <= 8) return launch_inorder_small<8, DUAL>(g, s);
-        if (g.n <= 16) return launch_inorder_small<16, DUAL>(g, s);
-        if (g.n <= 32) return launch_inorder_small<32, DUAL>(g, s);
-        if constexpr (DUAL) return launch_inorder_rows<1, 32, DUAL>(g, s);
-        return launch_inorder_small<64, DUAL>(g, s);
+void launch_chain(const GemmArgs& g, hipStream_t s) {
+    if (g.n <= 16) {
+        if (g.m <= 32768) return launch_chain_kt<1, 1, 1, 1, 64, DUAL>(g, s);
+        return launch_chain_kt<2, 1, 4, 1, 32, DUAL>(g, s);
     }
-    if (g.n > 32) {
-        // the 8x8 register-blocked kernel; 128-bit A loads at dword addresses
-        auto aligned = [](const float* p, int64_t) {
-            return p == nullptr || (reinterpret_cast<uintptr_t>(p) & 3) == 0;
-        };
-        const bool va4 = aligned(g.a1, g.lda1) && (!DUAL || aligned(g.a2, g.lda2));
-        dim3 grid(static_cast<unsigned>(ceil_div(g.m, kWBM)),
-                  static_cast<unsigned>(ceil_div(g.n, kWBN)));
-        if (va4)
-            gemm_inorder_wide_kernel<4, DUAL><<<grid, 256, 0, s>>>(g);
-        else
-            gemm_inorder_wide_kernel<1, DUAL><<<grid, 256, 0, s>>>(g);
-        TG_LAUNCH_CHECK();
-        return;
+    if (g.n <= 32) {
+        if (g.m <= 8192) return launch_chain_kt<1, 1, 1, 2, 64, DUAL>(g, s);
+        return launch_chain_kt<1, 2, 4, 1, 32, DUAL>(g, s);
     }
-    if (g.n > 16) return launch_inorder<128, 32, 4, 4, DUAL>(g, s);
-    if (g.n > 8 || DUAL) return launch_inorder<256, 16, 4, 4, DUAL>(g, s);
-    return launch_inorder<256, 8, 4, 2, DUAL>(g, s);
+    if (g.m * ceil_div(g.n, 64) <= 16384) return launch_chain_kt<1, 1, 1, 4, 64, DUAL>(g, s);
+    if (g.k1 * (DUAL ? 2 : 1) < 32) return launch_chain_kt<2, 2, 2, 2, 16, DUAL>(g, s);
+    launch_chain_as<2, 2, 2, 2, 32, DUAL, true>(g, s);
+}
+
+// The dual product in order: the columns before tail_from, then the tail's.
+void launch_chain_dual(const GemmArgs& g, hipStream_t s) {
+    require(g.k1 == g.k2, "matmul: the in-order dual product needs equal k");
+    require(g.tail_from < 0 || g.tail_from % 8 == 0,
+            "matmul: the dual product's tail columns must start at a multiple of 8");
+    const int64_t cut = g.tail_from >= 0 && g.tail_from < g.n ? g.tail_from : g.n;
+    if (cut > 0) {
+        GemmArgs h = g;
+        h.n = cut;
+        launch_chain<true>(h, s);
+    }
+    if (cut == g.n) return;
+    require(g.n - cut <= kDTCols && g.c_tile_stride == 0,
+            "matmul: at most 8 tail columns, of a row-major product");
+    GemmArgs h = g;
+    h.n = g.n - cut;
+    if (h.b1) h.b1 += cut;
+    if (h.b2) h.b2 += cut;
+    if (h.bias) h.bias += cut;
+    h.c += cut;
+    gemm_dual_tail_kernel<<<static_cast<unsigned>(ceil_div(g.m, kDTRows)), 256, 0, s>>>(h);
+    TG_LAUNCH_CHECK();
 }
 
 void unary_launch(int op, float* x, int64_t n, float alpha, hipStream_t s) {
@@ -1126,6 +969,13 @@ int resolve_gemm_algo(int algo, int64_t m, int64_t n, int64_t k) {
     return algo;
 }
 
+// Where AUTO may regroup the k order, the 128 x 128 tiles of gemm_mfma_kernel
+// pay from this many products on; below, their last wave leaves most of the
+// chip idle and the smaller tiles of gemm_chain_kernel are faster: 100,000 x
+// 512 x 128 (2^32.6) 139 against 155 us, 100,003 x 257 x 121 91 / 115, but
+// 500,000 x 256 x 256 (2^34.9) 692 / 616 and 232,965 x 602 x 256 697 / 645.
+constexpr int64_t kMfmaTilesOps = int64_t(1) << 33;
+
 void gemm(const GemmArgs& g, int algo, hipStream_t s) {
     require(g.m >= 0 && g.n >= 0 && g.k1 >= 0 && g.k2 >= 0, "matmul: negative dimension");
     require(g.epi == TG_EPI_NONE || g.epi == TG_EPI_RELU || g.epi == TG_EPI_ELU,
@@ -1142,7 +992,14 @@ void gemm(const GemmArgs& g, int algo, hipStream_t s) {
     const bool dual = g.a2 != nullptr;
     if (dual)
         require(g.b2 && g.lda2 >= g.k2 && g.ldb2 >= g.n, "matmul: bad second operand pair");
+    const int64_t ops = g.m * g.n * (g.k1 + g.k2);
+    const bool chain_fits = !dual || g.k1 == g.k2;
+    const bool any_order = algo == TG_GEMM_AUTO;
     algo = resolve_gemm_algo(algo, g.m, g.n, g.k1 + g.k2);
+    if (any_order && algo == TG_GEMM_MFMA && g.n >= 64 && chain_fits && ops < kMfmaTilesOps) {
+        if (!dual) return launch_chain<false>(g, s);
+        return launch_chain<true>(g, s);  // as one chain, without scalar-tail columns
+    }
     if (algo == TG_GEMM_MFMA && g.n <= 64) {
         // thin: one wavefront per 64 rows, 16-column MFMA tiles up to n
         const unsigned grid = static_cast<unsigned>(ceil_div(g.m, 256));
@@ -1202,13 +1059,8 @@ void gemm(const GemmArgs& g, int algo, hipStream_t s) {
 #undef TG_MFMA_CASE
         throw std::logic_error("matmul: no MFMA kernel for this access width");
     }
-    if (dual) {
-        require(g.k1 == g.k2, "matmul: the in-order dual product needs equal k");
-        require(g.tail_from < 0 || g.tail_from % 8 == 0,
-                "matmul: the dual product's tail columns must start at a multiple of 8");
-        return dispatch_inorder<true>(g, s);
-    }
-    dispatch_inorder<false>(g, s);
+    if (dual) return launch_chain_dual(g, s);
+    launch_chain<false>(g, s);
 }
 
 void add_bias_act(float* x, int64_t rows, int64_t cols, int64_t ld, const float* bias, int act,

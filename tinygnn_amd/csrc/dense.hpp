@@ -45,7 +45,7 @@ struct GemmArgs {
     int64_t c_tile_stride = 0;
 };
 
-// Resolves TG_GEMM_AUTO: MFMA when n >= 64 and k >= 32, else in order.
+// Resolves TG_GEMM_AUTO: any order (MFMA) for large products, else in order.
 int resolve_gemm_algo(int algo, int64_t m, int64_t n, int64_t k);
 void gemm(const GemmArgs& g, int algo, hipStream_t s);
 
