@@ -1475,12 +1475,20 @@ __global__ __launch_bounds__(256) void agg_reduce_kernel(const int4* __restrict_
 }
 
 // Column tile of the long-row kernel: the lane groups' tile when they are
-// given (column-blocked passes), else 32, 64 or 128 columns by f.
-inline int long_tile(int64_t f, const LaneLayout& L) {
-    if (L.tile == 32 || L.tile == 64 || L.tile == 128) {
-        if (L.n_tiles > 1 || L.tile >= f) return L.tile;
-    }
-    return f <= 32 ? 32 : f <= 64 ? 64 : 128;
+// given (column-blocked passes), else 32, 64 or 128 columns by f; narrower
+// where the rows have fewer than 128 workgroups, so that a row's gathers are
+// spread over more compute units (every column's chain is the same in any
+// tile).  100,000 rows of mean degree 5, the few split ones of up to 10,000
+// entries: SpMM at 100 columns 213 -> 160 us, at 256 246 -> 192; SAGE-Max
+// 256 -> 128 on it 405 -> 377.  With 512 in place of 128, 16,000 rows of mean
+// degree 100 took 105 us in place of 93 (100 columns): there enough rows are
+// long to fill the chip, and wider tiles gather longer runs.
+inline int long_tile(int64_t f, const LaneLayout& L, int64_t n_split) {
+    int tw = f <= 32 ? 32 : f <= 64 ? 64 : 128;
+    if ((L.tile == 32 || L.tile == 64 || L.tile == 128) && (L.n_tiles > 1 || L.tile >= f))
+        tw = L.tile;
+    while (tw > 32 && n_split * ceil_div(f, tw) < 128) tw /= 2;
+    return tw;
 }
 
 // Rows of more than one chunk summed as ONE chain each, in nonzero order:
@@ -1694,7 +1702,7 @@ void launch_agg(const PlanView& p, const LaneLayout& L, int64_t f, const int32_t
         if constexpr (MODE == kAggAttn) {
             throw std::logic_error("aggregate: long rows do not take attention weights");
         } else {
-            launch_long<VEC, MODE>(p, long_tile(f, L), f, ci, av, B, ldb, C, ldc, epi, s);
+            launch_long<VEC, MODE>(p, long_tile(f, L, p.n_split), f, ci, av, B, ldb, C, ldc, epi, s);
         }
     }
     if (p.n_chunks > 0) {
@@ -1723,7 +1731,7 @@ void launch_agg_sidx(const PlanView& p, const LaneLayout& L, int64_t f, const fl
     const int64_t ldp = round_up(f, 4);
     const int64_t* dc = p.dev_counts;
     if (epi.long_rows && p.n_split > 0)
-        launch_long<4, kAggSumTail>(p, long_tile(f, L), f, nullptr, nullptr, B, ldb, C, ldc,
+        launch_long<4, kAggSumTail>(p, long_tile(f, L, p.n_split), f, nullptr, nullptr, B, ldb, C, ldc,
                                     epi, s);
     if (p.n_chunks > 0) {
         dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, GPB)),
