@@ -46,6 +46,29 @@ def test_spmm_widths_bitexact(gpu, restate, f):
     np.testing.assert_array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("n", [1, 3, 400, 17000])
+@pytest.mark.parametrize("f", [1, 3, 6, 15, 16, 17, 20, 32, 33, 36, 64, 65, 100, 128, 129])
+def test_spmm_small_plans_bitexact(gpu, restate, n, f):
+    """Few enough chunks go one to a wavefront: rows around the batches of 32
+    to 128 entries, empty rows, odd and padded widths, and (17,000 rows) the
+    sizes on either side of the rule, bit for bit; split rows under FAST keep
+    their regrouped sums."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(11 * n + f)
+    a = random_csr(rng, n, max(n, 50), avg_deg=8, max_deg=300, empty_frac=0.1 if n > 9 else 0.0)
+    b = rng.standard_normal((max(n, 50), f)).astype(np.float32)
+    want = restate.spmm(a, b)
+    got, _ = _run(gpu, a, b)
+    np.testing.assert_array_equal(bits(got), bits(want))
+    got, _ = _run(gpu, a, b, chunk=40, precision=tg.PRECISION_FAST)
+    short = np.diff(a.row_ptr) <= 40
+    np.testing.assert_array_equal(bits(got[short]), bits(want[short]))
+    # a regrouped sum of at most 300 products
+    scale = restate.spmm(type(a)(a.n_rows, a.n_cols, a.row_ptr, a.col_ind, np.abs(a.val)),
+                         np.abs(b))
+    assert (np.abs(got - want) <= 2 * 302 * 2.0 ** -24 * scale).all()
+
+
 @pytest.mark.parametrize("chunk", [1, 7, 64, 256])
 @pytest.mark.parametrize("f", [2, 3, 4, 41, 128, 512])
 def test_spmm_split_rows_exact(gpu, restate, f, chunk):

@@ -1690,6 +1690,149 @@ void launch_long(const PlanView& p, int tw, int64_t f, const int32_t* ci, const 
     throw std::logic_error("aggregate: no long-row kernel for this tile width");
 }
 
+// Small plans: a wavefront per (chunk, TW-column tile).  A lane group of
+// agg_chunk_kernel has 16 gathers in flight and the plan's longest chunk
+// decides when a small launch ends (2,708 rows, the longest of 270 entries,
+// 16 columns: 17 round trips to memory, 18 us).  Here the whole wavefront
+// gathers, BE = 2048 / TW entries at a time, the next BE in flight
+// in registers while lanes [0, TW) walk the batch from LDS, one column each:
+// every column's chain is agg_chunk_kernel's, in nonzero order.  The LDS
+// regions belong to one wavefront each, so no barrier of the workgroup is
+// needed (their trip counts differ).
+// Against agg_chunk_kernel, weighted SpMM, same bits, us: 2,708 rows x 4 entries x 16 columns 18 -> 11, 3,000 x 100 x 16 31 ->
+// 11, 1,000 x 250 x 64 46 -> 25, 8,000 x 60 x 32 39 -> 17, 32,000 x 40 x 16
+// 119 -> 59 (its rows over 1,024 entries included).
+template <int VEC, int TW, int MODE>
+__global__ __launch_bounds__(256) void agg_small_kernel(
+    const int4* __restrict__ chunks, int64_t n_chunks, const int32_t* __restrict__ ci,
+    const float* __restrict__ av, const float* __restrict__ B, int64_t ldb,
+    float* __restrict__ C, int64_t ldc, float* __restrict__ partials, int64_t ldp, int64_t f,
+    AggEpilogue epi) {
+    static_assert(MODE == kAggWeighted || MODE == kAggSum || MODE == kAggMax, "mode");
+    constexpr int G = TW / VEC;      // lanes per gathered entry
+    constexpr int R = kWave / G;     // entries per round
+    constexpr int U = 32 / VEC;      // rounds per batch
+    constexpr int BE = U * R;        // entries per batch
+    constexpr int LW = (BE + kWave - 1) / kWave;  // weights per lane
+    static_assert(R >= 1 && BE * TW == 2048, "batch shape");
+    __shared__ __align__(16) float rows_lds[4][BE * TW];
+    __shared__ float w_lds[4][LW * kWave];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int64_t cid = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    if (cid >= n_chunks) return;
+    const int4 ch = chunks[cid];
+    if (epi.long_rows && ch.w >= 0) return;  // a split row: agg_long_kernel's
+    float* const rows = rows_lds[wave];
+    float* const wts = w_lds[wave];
+    const int q = lane / G, p = lane % G;
+    const int64_t fbase = static_cast<int64_t>(blockIdx.y) * TW;
+    const int64_t fo = fbase + static_cast<int64_t>(p) * VEC;
+    // lanes past f load the tile's first vector (in bounds), never used
+    const char* bl = reinterpret_cast<const char*>(B + (fo < f ? fo : fbase));
+    const uint32_t pitch = static_cast<uint32_t>(ldb) * 4u;
+    const int64_t fj = fbase + lane;
+    const bool chain_lane = lane < TW && fj < f;
+    float acc = MODE == kAggMax ? -INFINITY : 0.0f;
+
+    if (ch.z > ch.y) {
+        // entries past the chunk's end repeat its last one (never walked)
+        int col[U];
+        float g[U][VEC], w[LW];
+        auto columns = [&](int base) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t e = static_cast<int64_t>(base) + u * R + q;
+                col[u] = ci[e < ch.z ? e : ch.z - 1];
+            }
+        };
+        auto gathers = [&](int base) {
+            if constexpr (MODE == kAggWeighted) {
+#pragma unroll
+                for (int i = 0; i < LW; ++i) {
+                    const int64_t e = static_cast<int64_t>(base) + i * kWave + lane;
+                    w[i] = av[e < ch.z ? e : ch.z - 1];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                load_vec<VEC>(reinterpret_cast<const float*>(
+                                  bl + static_cast<uint64_t>(static_cast<uint32_t>(col[u])) * pitch),
+                              g[u]);
+        };
+        columns(ch.y);
+        gathers(ch.y);
+        const int n = ch.z - ch.y;
+        for (int t = 0; t < n; t += BE) {
+            const bool more = n - t > BE;
+            if (more) columns(ch.y + t + BE);
+            if constexpr (MODE == kAggWeighted) {
+#pragma unroll
+                for (int i = 0; i < LW; ++i) wts[i * kWave + lane] = w[i];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) store_vec<VEC>(&rows[(u * R + q) * TW + p * VEC], g[u]);
+            // the wavefront's LDS stores before its reads
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (more) gathers(ch.y + t + BE);
+            if (chain_lane) {
+                const int cnt = more ? BE : n - t;
+                const float* d = rows + lane;
+                int e = 0;
+                for (; e + 16 <= cnt; e += 16) {
+#pragma unroll
+                    for (int k = 0; k < 16; ++k)
+                        acc = combine<MODE>(acc, d[(e + k) * TW],
+                                            MODE == kAggWeighted ? wts[e + k] : 1.0f);
+                }
+                for (; e < cnt; ++e)
+                    acc = combine<MODE>(acc, d[e * TW], MODE == kAggWeighted ? wts[e] : 1.0f);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    if (!chain_lane) return;
+    if (ch.w < 0) {
+        if (MODE == kAggMax && ch.z == ch.y) acc = 0.0f;  // an empty row (layers.cpp:377-380)
+        float x[1] = {acc};
+        finish_store<1>(x, ch.x, ch.z - ch.y, fj, f, C, ldc, epi, false);
+    } else {
+        partials[static_cast<int64_t>(ch.w) * ldp + fj] = acc;
+    }
+}
+
+// Whether a plan's chunks go one to a wavefront (agg_small_kernel): plain
+// passes over a plan whose chunk count the host knows, up to two column
+// tiles, and few enough of them.  Either side of the lines, agg_chunk_kernel
+// / agg_small_kernel, us: 64,000 rows of 5 entries at 16 columns 124 / 41,
+// at 64 114 / 99, but 100,000 at 100 156 / 212; 32-bit loads (7 columns):
+// 16,000 rows 53 / 48, 64,000 118 / 150; 256 columns: 3,000 rows of 100
+// entries 22 / 32 (a chunk has a whole wavefront there already).
+inline int64_t small_tile(int64_t f) { return f <= 16 ? 16 : f <= 32 ? 32 : 64; }
+inline bool small_plan(const PlanView& p, int64_t f, int vec, const AggEpilogue& epi) {
+    return p.dev_counts == nullptr && !epi.acc && !epi.skip_empty && !epi.ci16 &&
+           epi.b_tile_stride == 0 && f <= 128 &&
+           p.n_chunks * ceil_div(f, small_tile(f)) <= (vec == 4 ? 65536 : 16384);
+}
+
+template <int VEC, int MODE>
+void launch_small(const PlanView& p, int64_t f, const int32_t* ci, const float* av,
+                  const float* B, int64_t ldb, float* C, int64_t ldc, int64_t ldp,
+                  const AggEpilogue& epi, hipStream_t s) {
+    const int64_t tw = small_tile(f);
+    const dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, 4)),
+                    static_cast<unsigned>(ceil_div(f, tw)));
+#define TG_SMALL(TW_)                                                                    \
+    if (tw == TW_)                                                                       \
+        agg_small_kernel<VEC, TW_, MODE><<<grid, 256, 0, s>>>(                           \
+            p.chunks, p.n_chunks, ci, av, B, ldb, C, ldc, p.partials, ldp, f, epi);
+    TG_SMALL(16) TG_SMALL(32) TG_SMALL(64)
+#undef TG_SMALL
+    TG_LAUNCH_CHECK();
+}
+
 template <int VEC, int LPR, int VPL, int MODE>
 void launch_agg(const PlanView& p, const LaneLayout& L, int64_t f, const int32_t* ci,
                 const float* av, const float* B, int64_t ldb, float* C, int64_t ldc,
@@ -1705,7 +1848,13 @@ void launch_agg(const PlanView& p, const LaneLayout& L, int64_t f, const int32_t
             launch_long<VEC, MODE>(p, long_tile(f, L, p.n_split), f, ci, av, B, ldb, C, ldc, epi, s);
         }
     }
-    if (p.n_chunks > 0) {
+    bool small = false;
+    if constexpr (MODE == kAggWeighted || MODE == kAggSum || MODE == kAggMax)
+        if (p.n_chunks > 0 && small_plan(p, f, VEC, epi)) {
+            launch_small<VEC, MODE>(p, f, ci, av, B, ldb, C, ldc, ldp, epi, s);
+            small = true;
+        }
+    if (p.n_chunks > 0 && !small) {
         // grid.y = column tile: the workgroups resident at a time (dispatched
         // in x order) gather from one or two tiles of B
         dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, GPB)),
