@@ -227,3 +227,41 @@ def test_gat_uniform_attention_is_mean(gpu, restate):
     for i in range(n):
         cols = a.col_ind[a.row_ptr[i]:a.row_ptr[i + 1]]
         np.testing.assert_allclose(got[i], wh[cols].astype(np.float64).mean(0), atol=2e-5)
+
+
+@pytest.mark.parametrize("heads,f", [(1, 1), (1, 7), (1, 41), (2, 8), (8, 8), (1, 64), (3, 33)])
+def test_gat_wave_chunks(gpu, heads, f):
+    """Few chunks: a wavefront's lane groups share a chunk.  Row lengths
+    around their batches, split rows, and scores of -inf (weight 0; a row of
+    nothing else is NaN), against fp64."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(heads * 100 + f)
+    lens = np.array([0, 1, 7, 8, 9, 16, 17, 31, 33, 64, 65, 127, 129, 200, 400, 50, 50])
+    n, rp = lens.size, np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = rng.integers(0, n - 1, size=rp[-1]).astype(np.int32)
+    ci[rp[15] + 8:rp[15] + 48] = n - 1  # row 15: mostly the -inf node, whole batches of it
+    ci[rp[15]:rp[15] + 8] = 3
+    ci[rp[16]:rp[17]] = n - 1        # row 16: nothing else
+    wh = rng.standard_normal((n, heads * f)).astype(np.float32)
+    src = rng.standard_normal((n, heads)).astype(np.float32)
+    dst = (3 * rng.standard_normal((n, heads))).astype(np.float32)
+    dst[n - 1] = -np.inf
+    da = tg.DeviceCSR.from_numpy(n, n, rp, ci, np.ones(ci.size, np.float32))
+    for chunk in (0, 96):
+        plan = _plan(da, heads * f, chunk)
+        plan.set_precision(tg.PRECISION_FAST)
+        got = tg.gat_aggregate(plan, da, _t(gpu, wh), heads, f, _t(gpu, src),
+                               _t(gpu, dst)).cpu().numpy()
+        assert np.isnan(got[16]).all() and np.isfinite(got[:16]).all()
+        for i in range(16):
+            e = src[i].astype(np.float64) + dst[ci[rp[i]:rp[i + 1]]].astype(np.float64)
+            e = np.where(e >= 0, e, np.float32(0.2) * e)
+            p = np.exp(e - e.max(axis=0)) if len(e) else e
+            w = wh[ci[rp[i]:rp[i + 1]]].astype(np.float64).reshape(-1, heads, f)
+            s = np.maximum(p.sum(axis=0), 1e-300)[:, None]
+            want = (p[:, :, None] * w).sum(axis=0) / s
+            scale = (p[:, :, None] * np.abs(w)).sum(axis=0) / s
+            # at most 400 terms, each weight within a few ulp of an exponent
+            # of magnitude up to 32 (2^-24 * 32 absolute)
+            bound = (400 + 3 * 32 + 16) * 2.0 ** -24 * scale + 1e-30
+            assert (np.abs(got[i].reshape(heads, f) - want) <= bound).all(), i

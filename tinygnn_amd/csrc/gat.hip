@@ -373,14 +373,24 @@ __global__ __launch_bounds__(256) void gat_exact_kernel(GatArgs a) {
         if (ok[v]) gat_store<VEC>(a, row, fo[v], acc[v], 1.0f);
 }
 
-template <int VEC, int LPR, int VPL>
+// WAVE: a whole wavefront per chunk, for plans of few chunks (gat_wave), where
+// the longest chunk decides when the launch ends.  Its kWave / LPR lane groups
+// take the chunk's batches in turn, each with its own max, sum and
+// accumulator, merged at the end as gat_reduce_kernel merges chunks.
+// Its sums are shorter chains (a layer's error against 64 bits 3.5e-7 -> 1.7e-7
+// at 200 entries a row).  One layer of 16 features, us: 2,708 rows of 4 entries
+// and 8 heads x 8 48 -> 23, 1,000 of 200 x 1 x 7 114 -> 19, 8,000 of 60 x 1 x 64
+// 110 -> 43, 32,000 of 40 x 8 x 8 178 -> 80, 100,000 of 5 x 4 x 32 188 -> 140.
+template <int VEC, int LPR, int VPL, bool WAVE>
 __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
     constexpr int GPB = 256 / LPR;
+    constexpr int NG = WAVE ? kWave / LPR : 1;  // lane groups per chunk
     constexpr int U = VPL <= 2 ? 8 : 4;  // gathers in flight per lane
     constexpr int TILE = LPR * VPL * VEC;
     const int g = threadIdx.x / LPR;
     const int l = threadIdx.x % LPR;
-    const int64_t cid = static_cast<int64_t>(blockIdx.x) * GPB + g;
+    const int part = g % NG;  // this group's turn among the chunk's batches
+    const int64_t cid = static_cast<int64_t>(blockIdx.x) * (GPB / NG) + g / NG;
     if (cid >= a.n_chunks) return;
     const int4 ch = a.chunks[cid];
     const int row = ch.x, b = ch.y, e = ch.z;
@@ -421,7 +431,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
     // row 0 and are not accumulated).
     constexpr int CPL = U > LPR ? U / LPR : 1;
     constexpr int BE = LPR * CPL;
-    for (int base = b; base < e; base += BE) {
+    for (int base = b + part * BE; base < e; base += NG * BE) {
         int cl[CPL];
 #pragma unroll
         for (int j = 0; j < CPL; ++j) {
@@ -456,7 +466,10 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
                     ev[u][v] = lrelu(si[v] + ev[u][v], a.slope);
                     if (u < nv) mn = (mn < ev[u][v]) ? ev[u][v] : mn;
                 }
-                const float sc = expf(m[v] - mn);
+                // a group that has met -inf scores only (another may hold
+                // the row's max) adds their exp(-inf) = 0
+                const float mx = WAVE && mn == -INFINITY ? 0.0f : mn;
+                const float sc = expf(m[v] - mx);
                 m[v] = mn;
                 s[v] *= sc;
 #pragma unroll
@@ -464,7 +477,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const bool valid = u < nv;  // a select, not a branch
-                    const float p = expf(ev[u][v] - mn);
+                    const float p = expf(ev[u][v] - mx);
                     s[v] = valid ? s[v] + p : s[v];
 #pragma unroll
                     for (int k = 0; k < VEC; ++k) {
@@ -475,6 +488,33 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
             }
           }
         }
+    }
+
+    if constexpr (NG > 1) {
+#pragma unroll
+        for (int off = LPR; off < kWave; off <<= 1) {
+#pragma unroll
+            for (int v = 0; v < VPL; ++v) {
+                const float mo = __shfl_xor(m[v], off), so = __shfl_xor(s[v], off);
+                const float mn = (m[v] < mo) ? mo : m[v];
+                const float mx = mn == -INFINITY ? 0.0f : mn;
+                const float c = expf(m[v] - mx), co = expf(mo - mx);
+                s[v] = s[v] * c + so * co;
+                m[v] = mn;
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+                    acc[v][k] = acc[v][k] * c + __shfl_xor(acc[v][k], off) * co;
+            }
+        }
+        if (part != 0) return;
+        // no score above -inf: exp(-inf - -inf), as one group's pass
+#pragma unroll
+        for (int v = 0; v < VPL; ++v)
+            if (m[v] == -INFINITY && b < e) {
+                s[v] = NAN;
+#pragma unroll
+                for (int k = 0; k < VEC; ++k) acc[v][k] = NAN;
+            }
     }
 
     if (split) {
@@ -557,6 +597,10 @@ __global__ __launch_bounds__(256) void gat_average_kernel(const float* __restric
     out[i * ldo + j] = finish_val(s, nullptr, 0, TG_ACT_NONE, post, exact != 0);
 }
 
+// Whether chunks take a wavefront each (gat_chunk_kernel, WAVE): as far as
+// measured (there), it was the faster at every size.
+inline bool gat_wave(int64_t n_chunks, int lpr) { return lpr < kWave && n_chunks <= 131072; }
+
 template <int VEC, int LPR, int VPL>
 void launch_gat(const tg_spmm_plan_s& p, const LaneLayout& L, GatArgs& a, hipStream_t s) {
     constexpr int GPB = 256 / LPR;
@@ -571,9 +615,13 @@ void launch_gat(const tg_spmm_plan_s& p, const LaneLayout& L, GatArgs& a, hipStr
         return;
     }
     if (p.n_chunks > 0) {
-        dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, GPB)),
+        const bool wave = gat_wave(p.n_chunks, LPR);
+        dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, wave ? 256 / kWave : GPB)),
                   static_cast<unsigned>(L.n_tiles));
-        gat_chunk_kernel<VEC, LPR, VPL><<<grid, 256, 0, s>>>(a);
+        if (wave)
+            gat_chunk_kernel<VEC, LPR, VPL, true><<<grid, 256, 0, s>>>(a);
+        else
+            gat_chunk_kernel<VEC, LPR, VPL, false><<<grid, 256, 0, s>>>(a);
         TG_LAUNCH_CHECK();
     }
     if (p.n_split > 0) {
