@@ -21,6 +21,8 @@
  * stay valid until the stream reaches the call.  Entry points that must
  * report a data-dependent error the reference raises (edge_list_to_csr's
  * endpoint check, CSR validation) synchronise the stream, and say so.
+ * A call that is given no workspace (NULL) does not wait for its end either:
+ * its temporaries are the library's, reused in stream order.
  */
 #ifndef TINYGNN_AMD_H
 #define TINYGNN_AMD_H

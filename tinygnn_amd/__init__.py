@@ -37,6 +37,18 @@ def stream_handle(stream=None) -> int:
     return int(s.cuda_stream)
 
 
+def _finish(stream) -> None:
+    """Waits for `stream` where it is not the current one.  The outputs of a
+    call are torch's memory of the current stream: reading a result's size, the
+    caller's next operation and the allocator's reuse of what the caller drops
+    are all ordered there, not after another stream's kernels."""
+    torch = _torch()
+    if stream is None or int(stream.cuda_stream) == int(torch.cuda.current_stream().cuda_stream):
+        return
+    wait = getattr(stream, "synchronize", None)
+    (wait or torch.cuda.ExternalStream(int(stream.cuda_stream)).synchronize)()
+
+
 def dptr(t, dtype=None) -> int:
     """Device pointer of a CUDA/HIP torch tensor (0 for None): contiguous, or
     a row-major 2-D view with unit column stride (its row stride is passed as
@@ -172,7 +184,8 @@ def spmm(a: DeviceCSR, b, plan: SpmmPlan | None = None, out=None, stream=None,
 # Graph preprocessing
 # ---------------------------------------------------------------------------
 def edge_list_to_csr(src, dst, n_nodes: int, stream=None) -> DeviceCSR:
-    """GraphLoader::edge_list_to_csr (graph_loader.cpp:211-281) on the device."""
+    """GraphLoader::edge_list_to_csr (graph_loader.cpp:211-281) on the device.
+    Given a `stream` that is not the current one, returns finished arrays."""
     torch = _torch()
     dev = src.device
     e = int(src.numel())
@@ -182,6 +195,7 @@ def edge_list_to_csr(src, dst, n_nodes: int, stream=None) -> DeviceCSR:
     lib.check(lib.tg_edge_list_to_csr(n_nodes, e, dptr(src, torch.int32), dptr(dst, torch.int32),
                                       dptr(rp), ci.data_ptr(), v.data_ptr(), None, 0,
                                       stream_handle(stream)))
+    _finish(stream)
     return DeviceCSR(n_nodes, n_nodes, rp, ci, v)
 
 
@@ -205,23 +219,26 @@ def _self_loop_outputs(a: DeviceCSR):
             torch.empty(max(cap, 1), dtype=torch.float32, device=dev))
 
 
-def _trim(a: DeviceCSR, rp, ci, v) -> DeviceCSR:
+def _trim(a: DeviceCSR, rp, ci, v, stream) -> DeviceCSR:
+    _finish(stream)
     nnz = int(rp[-1].item()) if a.n_rows else 0
     return DeviceCSR(a.n_rows, a.n_cols, rp, ci[:nnz], v[:nnz])
 
 
 def add_self_loops(a: DeviceCSR, stream=None) -> DeviceCSR:
-    """add_self_loops (layers.cpp:71-144): A + I, bit-identical structure/values."""
+    """add_self_loops (layers.cpp:71-144): A + I, bit-identical structure/values.
+    Waits for `stream`, whose result's size it reads."""
     _require_square(a, "add_self_loops")
     rp, ci, v = _self_loop_outputs(a)
     lib.check(lib.tg_add_self_loops(a.n_rows, a.nnz, dptr(a.row_ptr), a.col_ind.data_ptr(),
                                     a.val.data_ptr(), dptr(rp), dptr(ci), dptr(v), None, 0,
                                     stream_handle(stream)))
-    return _trim(a, rp, ci, v)
+    return _trim(a, rp, ci, v, stream)
 
 
 def gcn_norm(a: DeviceCSR, with_degrees: bool = False, stream=None):
-    """gcn_norm (layers.cpp:158-208): D^-1/2 (A+I) D^-1/2."""
+    """gcn_norm (layers.cpp:158-208): D^-1/2 (A+I) D^-1/2.  Waits for `stream`,
+    whose result's size it reads."""
     torch = _torch()
     _require_square(a, "gcn_norm")
     rp, ci, v = _self_loop_outputs(a)
@@ -230,7 +247,7 @@ def gcn_norm(a: DeviceCSR, with_degrees: bool = False, stream=None):
     lib.check(lib.tg_gcn_norm(a.n_rows, a.nnz, dptr(a.row_ptr), a.col_ind.data_ptr(),
                               a.val.data_ptr(), dptr(rp), dptr(ci), dptr(v), dptr(deg), dptr(dis),
                               None, 0, stream_handle(stream)))
-    out = _trim(a, rp, ci, v)
+    out = _trim(a, rp, ci, v, stream)
     return (out, deg[:a.n_rows], dis[:a.n_rows]) if with_degrees else out
 
 
@@ -328,7 +345,8 @@ def sage_aggregate(plan: SpmmPlan, a: DeviceCSR, h, agg: int = AGG_MEAN, stream=
 def sage_forward(plan: SpmmPlan, a: DeviceCSR, h, w_neigh, w_self, bias=None,
                  act: int = ACT_RELU, post: int = POST_NONE, agg: int = AGG_MEAN,
                  dataflow: int = SAGE_AUTO, stream=None):
-    """SAGELayer::forward (layers.cpp:538-752)."""
+    """SAGELayer::forward (layers.cpp:538-752).  Given a `stream` that is not
+    the current one, returns a finished result."""
     torch = _torch()
     f_in, f_out = w_neigh.shape
     out = torch.empty((a.n_rows, f_out), dtype=torch.float32, device=h.device)
@@ -336,6 +354,7 @@ def sage_forward(plan: SpmmPlan, a: DeviceCSR, h, w_neigh, w_self, bias=None,
                                   a.col_ind.data_ptr(), dptr(h), dptr(w_neigh), dptr(w_self),
                                   dptr(bias), act, post, dataflow, dptr(out), None, 0,
                                   stream_handle(stream)))
+    _finish(stream)
     return out
 
 
@@ -352,7 +371,8 @@ def gat_scores(wh, heads: int, f: int, att_l, att_r, stream=None):
 def gat_aggregate(plan: SpmmPlan, a_sl: DeviceCSR, wh, heads: int, f: int, src, dst,
                   slope: float = 0.2, bias=None, act: int = ACT_NONE, post: int = POST_NONE,
                   concat: bool = True, stream=None):
-    """All heads of GATLayer::forward's fused edge pass (layers.cpp:1052-1112)."""
+    """All heads of GATLayer::forward's fused edge pass (layers.cpp:1052-1112).
+    Given a `stream` that is not the current one, returns a finished result."""
     torch = _torch()
     cols = heads * f if (concat or heads == 1) else f
     out = torch.empty((a_sl.n_rows, cols), dtype=torch.float32, device=wh.device)
@@ -360,6 +380,7 @@ def gat_aggregate(plan: SpmmPlan, a_sl: DeviceCSR, wh, heads: int, f: int, src, 
                                    a_sl.col_ind.data_ptr(), dptr(wh), wh.stride(0), dptr(src),
                                    dptr(dst), slope, dptr(bias), act, post, int(concat),
                                    dptr(out), out.stride(0), None, 0, stream_handle(stream)))
+    _finish(stream)
     return out
 
 
