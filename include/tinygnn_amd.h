@@ -22,7 +22,8 @@
  * report a data-dependent error the reference raises (edge_list_to_csr's
  * endpoint check, CSR validation) synchronise the stream, and say so.
  * A call that is given no workspace (NULL) does not wait for its end either:
- * its temporaries are the library's, reused in stream order.
+ * its temporaries are the library's, reused in stream order.  On a stream
+ * under capture it fails with TG_ERR_INVALID_ARGUMENT.
  */
 #ifndef TINYGNN_AMD_H
 #define TINYGNN_AMD_H

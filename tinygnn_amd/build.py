@@ -12,6 +12,8 @@
   reference driven through the C++ API (tests/cpp/throw_sites.cpp).
 * ``tinygnn_amd/_build/test_numparse`` -- the CSV number conversions checked
   against the host C library (tests/cpp/test_numparse.cpp).
+* ``tinygnn_amd/_build/test_temporaries`` -- the library's temporary memory
+  over a stand-in for the HIP runtime (tests/cpp/test_temporaries.cpp).
 
 Usage: ``python -m tinygnn_amd.build [-j N] [--quiet]``.
 """
@@ -35,6 +37,7 @@ API_LIB = os.path.join(BUILD, "libtinygnn.so")
 CPP_TEST = os.path.join(BUILD, "test_cpp_api")
 THROW_TEST = os.path.join(BUILD, "test_throw_sites")
 NUMPARSE_TEST = os.path.join(BUILD, "test_numparse")
+TEMPORARIES_TEST = os.path.join(BUILD, "test_temporaries")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
@@ -106,6 +109,10 @@ def _build_cpp_api() -> None:
     _run(["g++", "-O2", "-std=c++17", "-Wall", f"-I{CSRC}",
           os.path.join(ROOT, "tests", "cpp", "test_numparse.cpp"), "-o", tmp])
     os.replace(tmp, NUMPARSE_TEST)
+    tmp = TEMPORARIES_TEST + ".tmp"
+    _run(host + [f"-I{CSRC}", os.path.join(ROOT, "tests", "cpp", "test_temporaries.cpp"), "-o",
+                 tmp, f"-L{BUILD}", "-ltinygnn_amd", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, TEMPORARIES_TEST)
 
 
 def _build_pybind() -> None:

@@ -83,10 +83,14 @@ void TempBuffer::allocate(size_t bytes, hipStream_t s) {
     reset();
     if (bytes == 0) return;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool keep = hipStreamIsCapturing(s, &capture) == hipSuccess &&
-                      capture == hipStreamCaptureStatusNone &&
-                      hipGetDevice(&device_) == hipSuccess && device_ >= 0 &&
-                      device_ < kMaxDevices;
+    const bool known = hipStreamIsCapturing(s, &capture) == hipSuccess;
+    // a graph would hold an address that is freed when the call returns (a
+    // capture in relaxed mode lets hipMalloc and hipFree through)
+    require(!known || capture == hipStreamCaptureStatusNone,
+            "the stream is being captured and this call allocates its temporaries: pass it a "
+            "workspace, or make it outside the capture");
+    const bool keep =
+        known && hipGetDevice(&device_) == hipSuccess && device_ >= 0 && device_ < kMaxDevices;
     if (!keep) (void)hipGetLastError();
     const size_t want = keep ? block_size(bytes) : bytes;
     if (keep) {

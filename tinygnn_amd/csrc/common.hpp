@@ -131,8 +131,7 @@ private:
 // 100 MB workspace on every call cost a SAGE-Max layer of 100K nodes 5.3 of its
 // 5.8 ms.  (A hipMemPool's hipFreeAsync took 8 to 20 us of host time each, and
 // after some hundred loads of a 5M-edge graph the pool went to the driver on
-// every one: 1.7 ms a load, then 4.7.)  Where s is being captured the memory
-// comes from hipMalloc, which capture refuses.
+// every one: 1.7 ms a load, then 4.7.)  A stream under capture is refused.
 class TempBuffer {
 public:
     TempBuffer() = default;
