@@ -67,6 +67,12 @@ const char* tg_last_error(void);
 /* Library version, (major << 16) | minor. */
 int tg_version(void);
 
+/* Gives the memory that the library keeps for the temporaries of later calls
+ * (at most 512 MiB per device) back to the driver, for other allocators and
+ * before a hipDeviceReset.  Waits for the devices that hold some; the
+ * library's own allocations do it by themselves before they fail. */
+int tg_trim(void);
+
 /* ------------------------------------------------------------------------
  * CSR construction -- replaces GraphLoader::edge_list_to_csr
  * (src/graph_loader.cpp:211-281, include/tinygnn/graph_loader.hpp:74-76).

@@ -132,11 +132,40 @@ void blocks_are_reused() {
     g_waits.clear();
 }
 
+// Kept blocks are no reason for another allocation of the library to fail, and
+// a program can have them back.
+void kept_blocks_are_given_back() {
+    expect(g_bytes > 100 * kMiB, "some memory kept");
+    g_limit = g_bytes + kMiB;
+    {
+        tg::DeviceBuffer d;
+        bool failed = false;
+        try {
+            d.resize(64 * kMiB);
+        } catch (const tg::AllocError&) {
+            failed = true;
+        }
+        expect(!failed, "a plan's allocation takes the kept memory back");
+        try {
+            d.resize(g_limit + kMiB);
+        } catch (const tg::AllocError&) {
+            failed = true;
+        }
+        expect(failed && d.get() == nullptr && d.size() == 0, "one that cannot be met fails");
+    }
+    {
+        tg::TempBuffer t(8 * kMiB, kA);
+    }
+    expect(g_bytes == 8 * kMiB, "kept");
+    expect(tg_trim() == TG_OK && g_bytes == 0 && g_live.empty(), "given back on request");
+}
+
 }  // namespace
 
 int main() {
     capture_is_refused();
     blocks_are_reused();
+    kept_blocks_are_given_back();
     std::printf(g_failures ? "%d failed\n" : "ok\n", g_failures);
     return g_failures != 0;
 }

@@ -17,6 +17,25 @@ def test_kept_blocks_on_the_host():
 
 
 @pytest.mark.gpu
+def test_trim(gpu):
+    """What a call's temporaries leave behind goes back to the driver."""
+    import tinygnn_amd as tg
+    torch = gpu
+    n = 100_000
+    d = tg.DeviceCSR(n, n, torch.arange(n + 1, dtype=torch.int32, device="cuda"),
+                     torch.arange(n, dtype=torch.int32, device="cuda"),
+                     torch.ones(n, device="cuda"))
+    plan = tg.SpmmPlan(d.row_ptr, n, n, 256)
+    x, w = torch.ones(n, 256, device="cuda"), torch.ones(256, 64, device="cuda")
+    out = tg.sage_forward(plan, d, x, w, w, dataflow=tg.SAGE_CONCAT)  # 100 MB of its own
+    torch.cuda.synchronize()
+    kept = torch.cuda.mem_get_info()[0]
+    tg.trim()
+    assert torch.cuda.mem_get_info()[0] - kept >= 4 * n * 256
+    assert float(out[0, 0]) == 512.0
+
+
+@pytest.mark.gpu
 def test_capture_needs_a_workspace(gpu, restate):
     """Under capture, in a mode that would let hipMalloc through, a call that
     would allocate is refused and the capture goes on; with a workspace it is

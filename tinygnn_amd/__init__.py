@@ -49,6 +49,12 @@ def _finish(stream) -> None:
     (wait or torch.cuda.ExternalStream(int(stream.cuda_stream)).synchronize)()
 
 
+def trim() -> None:
+    """Gives the memory kept for the temporaries of later calls (at most 512
+    MiB per device) back to the driver, for other allocators."""
+    lib.check(lib.tg_trim())
+
+
 def dptr(t, dtype=None) -> int:
     """Device pointer of a CUDA/HIP torch tensor (0 for None): contiguous, or
     a row-major 2-D view with unit column stride (its row stride is passed as

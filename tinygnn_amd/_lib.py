@@ -58,6 +58,7 @@ class OutOfRange(TgError, IndexError):
 SIGNATURES = {
     "tg_last_error": (C.c_char_p, []),
     "tg_version": (i32, []),
+    "tg_trim": (i32, []),
     "tg_edge_list_to_csr_workspace_size": (sz, [i64, i64]),
     "tg_edge_list_to_csr": (i32, [i64, i64, vp, vp, vp, vp, vp, vp, sz, vp]),
     "tg_csr_validate": (i32, [i64, i64, i64, vp, vp, vp]),

@@ -91,6 +91,10 @@ struct DevBuf {
         release();
         if (bytes == 0) bytes = 4;
         hipError_t e = hipMallocFromPoolAsync(&p, bytes, library_pool(), nullptr);
+        if (e == hipErrorOutOfMemory && tg_trim() == TG_OK) {  // what the C library keeps, given back
+            (void)hipGetLastError();
+            e = hipMallocFromPoolAsync(&p, bytes, library_pool(), nullptr);
+        }
         if (e != hipSuccess) hip_fail(e, "hipMallocFromPoolAsync");
         n = bytes;
     }

@@ -24,25 +24,6 @@ void throw_hip(hipError_t e, const char* what, const char* file, int line) {
     throw HipError(msg);
 }
 
-void DeviceBuffer::resize(size_t bytes) {
-    reset();
-    if (bytes == 0) return;
-    hipError_t e = hipMalloc(&p_, bytes);
-    if (e != hipSuccess) {
-        p_ = nullptr;
-        (void)hipGetLastError();
-        throw AllocError("hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
-                         hipGetErrorString(e));
-    }
-    n_ = bytes;
-}
-
-void DeviceBuffer::reset() {
-    if (p_) (void)hipFree(p_);
-    p_ = nullptr;
-    n_ = 0;
-}
-
 namespace {
 
 constexpr size_t kKeepBytes = size_t(512) << 20;
@@ -71,6 +52,36 @@ void give_back(const Block& b) {
     (void)hipEventDestroy(b.event);
 }
 
+// Gives a device's kept blocks back to the driver: whether there were any.
+bool give_back_kept(int device) {
+    std::vector<Block> old;
+    {
+        Blocks& bl = blocks_of(device);
+        std::lock_guard<std::mutex> lock(bl.mu);
+        old.swap(bl.list);
+        bl.bytes = 0;
+    }
+    for (const Block& b : old) give_back(b);
+    return !old.empty();
+}
+
+// hipMalloc on the current device; where that fails for want of memory that
+// the kept blocks hold, once more without them.
+hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    int device = -1;
+    if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && device >= 0 &&
+        device < kMaxDevices) {
+        (void)hipGetLastError();
+        if (give_back_kept(device)) e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+    }
+    return e;
+}
+
 // Sizes of a call vary a little from one to the next: whole 64 KB, or 2 MB.
 size_t block_size(size_t bytes) {
     const size_t unit = bytes <= (size_t(1) << 20) ? size_t(64) << 10 : size_t(2) << 20;
@@ -78,6 +89,22 @@ size_t block_size(size_t bytes) {
 }
 
 }  // namespace
+
+void DeviceBuffer::resize(size_t bytes) {
+    reset();
+    if (bytes == 0) return;
+    const hipError_t e = device_malloc(&p_, bytes);
+    if (e != hipSuccess)
+        throw AllocError("hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
+                         hipGetErrorString(e));
+    n_ = bytes;
+}
+
+void DeviceBuffer::reset() {
+    if (p_) (void)hipFree(p_);
+    p_ = nullptr;
+    n_ = 0;
+}
 
 void TempBuffer::allocate(size_t bytes, hipStream_t s) {
     reset();
@@ -132,30 +159,20 @@ void TempBuffer::allocate(size_t bytes, hipStream_t s) {
             TG_HIP(e);
         }
     }
-    hipError_t e = hipMalloc(&p_, want);
-    if (e != hipSuccess && keep) {  // give the kept blocks back, then once more
-        (void)hipGetLastError();
-        std::vector<Block> old;
-        {
-            Blocks& bl = blocks_of(device_);
-            std::lock_guard<std::mutex> lock(bl.mu);
-            old.swap(bl.list);
-            bl.bytes = 0;
-        }
-        for (const Block& b : old) give_back(b);
-        e = hipMalloc(&p_, want);
-    }
+    const hipError_t e = device_malloc(&p_, want);
     if (e != hipSuccess) {
-        p_ = nullptr;
         if (event_) (void)hipEventDestroy(event_);
         event_ = nullptr;
-        (void)hipGetLastError();
         throw AllocError("hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
                          hipGetErrorString(e));
     }
     n_ = bytes;
     block_ = keep ? want : 0;
     stream_ = s;
+}
+
+void trim_memory() {
+    for (int d = 0; d < kMaxDevices; ++d) give_back_kept(d);
 }
 
 void TempBuffer::reset() {
@@ -348,5 +365,9 @@ extern "C" {
 const char* tg_last_error(void) { return tg::last_error(); }
 
 int tg_version(void) { return (0 << 16) | 1; }
+
+int tg_trim(void) {
+    return tg::guard([] { tg::trim_memory(); });
+}
 
 }  // extern "C"

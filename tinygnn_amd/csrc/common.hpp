@@ -125,8 +125,9 @@ private:
 
 // RAII device memory for a call's own temporaries, in stream order: freed
 // blocks are kept (per device, at most kKeepBytes, oldest given back first, all
-// of them before an allocation fails) with an event of the freeing stream, which
-// the next user's stream waits for where it is not past yet.  So a warm call
+// of them before an allocation of the library fails and by trim_memory) with an
+// event of the freeing stream, which the next user's stream waits for where it
+// is not past yet.  So a warm call
 // neither waits for the GPU nor enters the driver: hipMalloc and hipFree of a
 // 100 MB workspace on every call cost a SAGE-Max layer of 100K nodes 5.3 of its
 // 5.8 ms.  (A hipMemPool's hipFreeAsync took 8 to 20 us of host time each, and
@@ -157,6 +158,9 @@ private:
     hipEvent_t event_ = nullptr;
     bool idle_free_ = false;
 };
+
+// Gives every device's kept blocks back to the driver.
+void trim_memory();
 
 // RAII pinned host allocation (hipHostMalloc): small device-to-host results
 // that the host reads after a stream synchronisation, so that the copies
