@@ -20,6 +20,7 @@ std::vector<size_t> g_freed;
 std::set<hipEvent_t> g_pending;
 std::vector<std::pair<hipStream_t, hipEvent_t>> g_waits;
 hipStreamCaptureStatus g_capture = hipStreamCaptureStatusNone;
+hipError_t g_device_sync = hipSuccess;
 int g_failures = 0;
 
 void expect(bool ok, const char* what) {
@@ -51,6 +52,9 @@ hipError_t hipGetDevice(int* d) {
     *d = 0;
     return hipSuccess;
 }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { return g_device_sync; }
+hipError_t hipHostMalloc(void**, size_t, unsigned) { return hipErrorOutOfMemory; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
     *e = reinterpret_cast<hipEvent_t>(g_next++);
@@ -160,12 +164,28 @@ void kept_blocks_are_given_back() {
     expect(tg_trim() == TG_OK && g_bytes == 0 && g_live.empty(), "given back on request");
 }
 
+// A CSV handle's memory is kept, without an event, once its device is idle;
+// where the device cannot be waited for it goes to the driver.  (Opening fails
+// here at the pinned staging buffers, after the file's memory.)
+void handles_wait_for_the_device(const char* file) {
+    for (bool idle : {true, false}) {
+        g_device_sync = idle ? hipSuccess : hipErrorStreamCaptureUnsupported;
+        g_freed.clear();
+        tg_csv_t csv = nullptr;
+        expect(tg_csv_open(file, &csv, nullptr) == TG_ERR_ALLOC && csv == nullptr, "open fails");
+        expect(g_freed.empty() == idle, idle ? "kept when idle" : "to the driver when not");
+        expect(tg_trim() == TG_OK && g_live.empty(), "nothing left");
+    }
+    g_device_sync = hipSuccess;
+}
+
 }  // namespace
 
-int main() {
+int main(int, char** argv) {
     capture_is_refused();
     blocks_are_reused();
     kept_blocks_are_given_back();
+    handles_wait_for_the_device(argv[0]);
     std::printf(g_failures ? "%d failed\n" : "ok\n", g_failures);
     return g_failures != 0;
 }

@@ -145,6 +145,8 @@ public:
     // For memory that outlives the call (s may be gone by its end): the device
     // must be idle when it is freed.
     void outlive_stream() { idle_free_ = true; }
+    // To the driver when it is freed (which waits), not to the kept blocks.
+    void to_driver() { block_ = 0; }
     void* get() const { return p_; }
     template <typename T> T* as() const { return static_cast<T*>(p_); }
     size_t size() const { return n_; }

@@ -66,11 +66,15 @@ struct tg_csv_s {
         int now = device;
         (void)hipGetDevice(&now);
         if (now != device) (void)hipSetDevice(device);
-        (void)hipDeviceSynchronize();
+        if (hipDeviceSynchronize() != hipSuccess) {  // not known to be idle
+            (void)hipGetLastError();
+            for (tg::TempBuffer* b : {&own_text, &bounds, &fields}) b->to_driver();
+        }
         if (now != device) (void)hipSetDevice(now);
     }
     int device = 0;
     static void make(tg::TempBuffer& b, size_t bytes, hipStream_t s) {
+        b.to_driver();  // what a failed call left may be in use
         b.allocate(bytes, s);
         b.outlive_stream();
     }
