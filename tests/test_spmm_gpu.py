@@ -14,6 +14,7 @@ reference-order path.)
 import numpy as np
 import pytest
 
+import oracle
 from helpers import bits, random_csr
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +68,26 @@ def test_spmm_small_plans_bitexact(gpu, restate, n, f):
     scale = restate.spmm(type(a)(a.n_rows, a.n_cols, a.row_ptr, a.col_ind, np.abs(a.val)),
                          np.abs(b))
     assert (np.abs(got - want) <= 2 * 302 * 2.0 ** -24 * scale).all()
+
+
+@pytest.mark.parametrize("f", [7, 16, 64, 100, 128])
+@pytest.mark.parametrize("n,row,long", [(9000, 3, 0), (9000, 3, 93), (9000, 3, 94),
+                                        (9000, 3, 321), (9000, 3, 322), (9000, 3, 2500), (4200, 80, 0),
+                                        (4200, 80, 400), (1000, 100, 0), (12400, 70, 900)])
+def test_spmm_plan_shapes_bitexact(gpu, restate, n, row, long, f):
+    """Rows of one length beside one longer row, on either side of the lines
+    between a wavefront and a lane group per chunk: the same chains, bit for
+    bit."""
+    rng = np.random.default_rng(n + long + f)
+    deg = np.full(n, row)
+    if long:
+        deg[n // 3] = long
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    a = oracle.CSR(n, n, rp, rng.integers(0, n, rp[-1]).astype(np.int32),
+                   rng.standard_normal(rp[-1]).astype(np.float32))
+    b = rng.standard_normal((n, f)).astype(np.float32)
+    got, _ = _run(gpu, a, b)
+    np.testing.assert_array_equal(bits(got), bits(restate.spmm(a, b)))
 
 
 @pytest.mark.parametrize("chunk", [1, 7, 64, 256])

@@ -34,6 +34,10 @@ __device__ __forceinline__ int chunk_bin(int len) {
     return b < kPlanBins ? b : kPlanBins - 1;
 }
 
+// The chunks' last counter, past every length's bin (an int's ends at 61),
+// holds the longest row of one chunk instead.
+constexpr int kTopSlot = kPlanBins - 1;
+
 // bin_count holds 2 x kPlanBins counters: the chunks' length bins, then the
 // split rows' degree bins (split rows are listed longest first too).
 __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restrict__ row_ptr,
@@ -45,6 +49,7 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
     for (int i = threadIdx.x; i < 2 * kPlanBins; i += blockDim.x) hist[i] = 0;
     __syncthreads();
     const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    int top = 0;
     if (r < m) {
         const int deg = row_ptr[r + 1] - row_ptr[r];
         const int nch = deg <= chunk ? 1 : (deg + chunk - 1) / chunk;
@@ -52,6 +57,7 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
         is_split[r] = nch > 1 ? 1 : 0;
         if (nch == 1) {
             atomicAdd(&hist[chunk_bin(deg)], 1);
+            top = deg;
         } else {
             const int full = deg / chunk, rem = deg - full * chunk;
             atomicAdd(&hist[chunk_bin(chunk)], full);
@@ -59,15 +65,26 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
             atomicAdd(&hist[kPlanBins + chunk_bin(deg)], 1);
         }
     }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d, kWave));
+    if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(&hist[kTopSlot], top);
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * kPlanBins; i += blockDim.x)
-        if (hist[i]) atomicAdd(&bin_count[i], hist[i]);
+    for (int i = threadIdx.x; i < 2 * kPlanBins; i += blockDim.x) {
+        if (i == kTopSlot) {  // (few of the workgroups raise it)
+            if (hist[i] > __hip_atomic_load(&bin_count[i], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(&bin_count[i], hist[i]);
+        } else if (hist[i]) {
+            atomicAdd(&bin_count[i], hist[i]);
+        }
+    }
 }
 
 // Turns bin counts into start cursors, longest bin first; writes totals.
 // With caps (a plan built into fixed scratch), totals beyond the capacities
 // (a row_ptr inconsistent with the nnz the caller gave) zero the counts the
-// kernels read, so nothing runs, and set totals[3].
+// kernels read, so nothing runs, and set totals[3]; without, totals[3] is the
+// longest row of one chunk.
 __global__ void plan_bins_kernel(const int32_t* __restrict__ bin_count,
                                  int32_t* __restrict__ bin_cursor,
                                  const int32_t* __restrict__ slot_base,
@@ -76,7 +93,7 @@ __global__ void plan_bins_kernel(const int32_t* __restrict__ bin_count,
                                  int64_t cap_split, int64_t cap_partials) {
     if (threadIdx.x == 0) {
         int64_t acc = 0;
-        for (int b = kPlanBins - 1; b >= 0; --b) {
+        for (int b = kTopSlot - 1; b >= 0; --b) {
             bin_cursor[b] = static_cast<int32_t>(acc);
             acc += bin_count[b];
         }
@@ -90,7 +107,7 @@ __global__ void plan_bins_kernel(const int32_t* __restrict__ bin_count,
         totals[0] = over ? 0 : acc;      // chunks
         totals[1] = over ? 0 : n_split;  // split rows
         totals[2] = n_part;              // partial slots
-        totals[3] = over ? 1 : 0;
+        totals[3] = cap_chunks == INT64_MAX ? bin_count[kTopSlot] : over ? 1 : 0;
     }
 }
 
@@ -207,8 +224,8 @@ void build_plan_count(tg_spmm_plan_s& p, int64_t m, int64_t nnz_bound, const int
     p.max_f = max_f;
     p.chunk = chunk;
     p.row_ptr = row_ptr;
-    p.n_chunks = p.n_split = p.n_partials = 0;
-    host_totals[0] = host_totals[1] = host_totals[2] = 0;
+    p.n_chunks = p.n_split = p.n_partials = p.top = 0;
+    for (int i = 0; i < 4; ++i) host_totals[i] = 0;
     if (m == 0) return;
     require(row_ptr != nullptr, "spmm plan: row_ptr is null");
     const PlanTemps t = carve_plan_temps(p, m);
@@ -223,13 +240,14 @@ void build_plan_count(tg_spmm_plan_s& p, int64_t m, int64_t nnz_bound, const int
     plan_bins_kernel<<<1, 64, 0, s>>>(t.bin_count, t.bin_cursor, t.slot_base, t.split_pos, m,
                                       t.totals, kNoCap, kNoCap, kNoCap);
     TG_LAUNCH_CHECK();
-    TG_HIP(hipMemcpyAsync(host_totals, t.totals, 3 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    TG_HIP(hipMemcpyAsync(host_totals, t.totals, 4 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
 }
 
 void build_plan_finish(tg_spmm_plan_s& p, const int64_t* host_totals, hipStream_t s) {
     p.n_chunks = host_totals[0];
     p.n_split = host_totals[1];
     p.n_partials = host_totals[2];
+    p.top = host_totals[3];
     if (p.m == 0) return;
     const PlanTemps t = carve_plan_temps(p, p.m);
     p.chunks.reserve(static_cast<size_t>(std::max<int64_t>(p.n_chunks, 1)) * sizeof(int4));
@@ -439,6 +457,7 @@ void build_plans_multi(tg_spmm_plan_s* const* plans, int nplans, int64_t m,
         p.n_chunks = host_totals[4 * b + 0];
         p.n_split = host_totals[4 * b + 1];
         p.n_partials = host_totals[4 * b + 2];
+        p.top = 0;
         p.chunks.reserve(static_cast<size_t>(std::max<int64_t>(p.n_chunks, 1)) * sizeof(int4));
         p.split.reserve(static_cast<size_t>(std::max<int64_t>(p.n_split, 1)) * sizeof(int4));
         if (p.n_partials > 0 && p.max_f > 0)
@@ -1805,17 +1824,39 @@ __global__ __launch_bounds__(256) void agg_small_kernel(
 }
 
 // Whether a plan's chunks go one to a wavefront (agg_small_kernel): plain
-// passes over a plan whose chunk count the host knows, up to two column
-// tiles, and few enough of them.  Either side of the lines, agg_chunk_kernel
-// / agg_small_kernel, us: 64,000 rows of 5 entries at 16 columns 124 / 41,
-// at 64 114 / 99, but 100,000 at 100 156 / 212; 32-bit loads (7 columns):
-// 16,000 rows 53 / 48, 64,000 118 / 150; 256 columns: 3,000 rows of 100
-// entries 22 / 32 (a chunk has a whole wavefront there already).
+// passes over a plan whose counts the host knows, up to two column tiles.  A
+// lane group's time is the longest chunk's round trips, a wavefront's the
+// number of chunks (a batch is gathered whole), so the line is where the
+// longest chunk is long for the number of chunks.  agg_chunk_kernel /
+// agg_small_kernel, us (power-law rows unless noted):
+//   60,000 rows, longest 1,024: 97 / 65 at 16 columns, 86 / 74 at 64; 60,000
+//   rows of 3 entries each: 11 / 30, 16 / 36; 9,000, longest 900: 44 / 13, 28 /
+//   20.  Up to 8,192 tiles (4,096 of 32-bit loads) either runs in the time of
+//   the call, 11 on the host.  32-bit loads (7 columns): 16,000, longest 1,024,
+//   43 / 41, 64,000 118 / 150.
+// Where rows are long on average and alike, both are bound by the gathers, and
+// a batch's slack is lost: 16,000 of 200 each at 16 columns 23 / 29, 4,000 at 64
+// 14 / 16, at 7 15 / 18.  Two tiles gather 128 columns for f: 4,000 of 100
+// (longest 400) at 80 columns 20 / 25, 32,000 133 / 155; but 2,708 of 100 21 /
+// 16, and close to 128 columns a tile of B stays in an XCD's L2 where its rows
+// do not: 32,000 of 100 at 128 columns 176 / 151, of 100 each 174 / 136.  256
+// columns: 3,000 rows of 100 22 / 32 (a chunk has a whole wavefront there).
 inline int64_t small_tile(int64_t f) { return f <= 16 ? 16 : f <= 32 ? 32 : 64; }
 inline bool small_plan(const PlanView& p, int64_t f, int vec, const AggEpilogue& epi) {
-    return p.dev_counts == nullptr && !epi.acc && !epi.skip_empty && !epi.ci16 &&
-           epi.b_tile_stride == 0 && f <= 128 &&
-           p.n_chunks * ceil_div(f, small_tile(f)) <= (vec == 4 ? 65536 : 16384);
+    if (p.dev_counts != nullptr || epi.acc || epi.skip_empty || epi.ci16 ||
+        epi.b_tile_stride != 0 || f > 128)
+        return false;
+    const int64_t tiles = p.n_chunks * ceil_div(f, small_tile(f));
+    if (tiles > (vec == 4 ? 65536 : 16384)) return false;
+    const bool few = tiles <= (vec == 4 ? 8192 : 4096);
+    // the longest chunk of this launch (split rows: agg_long_kernel's, or cut)
+    const int64_t longest = p.n_split > 0 && !epi.long_rows ? p.chunk : p.top;
+    if (p.nnz >= 64 * p.n_chunks) {
+        if (f > 112 && p.n_chunks > 12288) return true;
+        if (f > 64 && p.nnz > 300000) return false;
+        if (longest * p.n_chunks < 2 * p.nnz) return few && f <= 32 && vec == 4;
+    }
+    return few || tiles <= (vec == 4 ? 96 : 28) * longest;
 }
 
 template <int VEC, int MODE>

@@ -24,6 +24,7 @@ struct tg_spmm_plan_s {
     int64_t n_chunks = 0;
     int64_t n_split = 0;
     int64_t n_partials = 0;
+    int64_t top = 0;     // entries of the longest row of one chunk (0: not counted)
     int device = 0;
     // summation order of the plan's executes: TG_PRECISION_EXACT (the
     // default) sums split rows as single in-order chains, TG_PRECISION_FAST
@@ -50,6 +51,8 @@ struct PlanView {
     int64_t max_f = 0;
     int64_t n_chunks = 0;
     int64_t n_split = 0;
+    // what a launch's shape is chosen by (0 with dev_counts)
+    int64_t nnz = 0, chunk = 0, top = 0;
     const int4* chunks = nullptr;
     const int4* split = nullptr;
     float* partials = nullptr;
@@ -63,6 +66,9 @@ inline PlanView plan_view(const tg_spmm_plan_s& p) {
     v.max_f = p.max_f;
     v.n_chunks = p.n_chunks;
     v.n_split = p.n_split;
+    v.nnz = p.nnz_bound;
+    v.chunk = p.chunk;
+    v.top = p.top;
     v.chunks = p.chunks.as<int4>();
     v.split = p.split.as<int4>();
     v.partials = p.partials.as<float>();
@@ -81,7 +87,7 @@ void build_plan(tg_spmm_plan_s& p, int64_t m, int64_t nnz_bound, const int32_t* 
 
 // The same build in two phases, so that several plans share one
 // synchronisation: build_plan_count enqueues the counting and the copy of
-// the three totals to host_totals (pinned host memory, 3 int64); once `s`
+// the four totals to host_totals (pinned host memory, 4 int64); once `s`
 // has synchronised, build_plan_finish sizes the plan and enqueues the
 // scatter.
 void build_plan_count(tg_spmm_plan_s& p, int64_t m, int64_t nnz_bound, const int32_t* row_ptr,
