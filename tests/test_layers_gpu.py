@@ -265,3 +265,46 @@ def test_gat_wave_chunks(gpu, heads, f):
             # of magnitude up to 32 (2^-24 * 32 absolute)
             bound = (400 + 3 * 32 + 16) * 2.0 ** -24 * scale + 1e-30
             assert (np.abs(got[i].reshape(heads, f) - want) <= bound).all(), i
+
+
+def _check_gat_rows(got, rows, rp, ci, wh, src, dst, heads, f):
+    """Rows of a GAT aggregation against fp64: at most max(len) terms, each
+    weight within a few ulp of an exponent of magnitude up to 32 (2^-24 * 32
+    absolute)."""
+    for i in rows:
+        c = ci[rp[i]:rp[i + 1]]
+        e = src[i].astype(np.float64) + dst[c].astype(np.float64)
+        e = np.where(e >= 0, e, np.float32(0.2) * e)
+        p = np.exp(e - e.max(axis=0))
+        w = wh[c].astype(np.float64).reshape(-1, heads, f)
+        s = p.sum(axis=0)[:, None]
+        want = (p[:, :, None] * w).sum(axis=0) / s
+        scale = (p[:, :, None] * np.abs(w)).sum(axis=0) / s
+        bound = (len(c) + 3 * 32 + 16) * 2.0 ** -24 * scale + 1e-30
+        assert (np.abs(got[i].reshape(heads, f) - want) <= bound).all(), i
+
+
+@pytest.mark.parametrize("heads,f", [(1, 7), (8, 4), (1, 64)])
+@pytest.mark.parametrize("n,long", [(9000, 70), (9000, 71), (131000, 2500), (131200, 2500)])
+def test_gat_wave_lines(gpu, heads, f, n, long):
+    """Rows of 1 to 3 entries and a few longer ones, on either side of the lines
+    between a wavefront and a lane group per chunk (9,000 chunks and the longest
+    of them; 131,072 chunks), against fp64."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(n + long + f)
+    lens = rng.integers(1, 4, size=n)
+    longs = rng.choice(n, size=4, replace=False)
+    lens[longs] = long
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = rng.integers(0, n, size=rp[-1]).astype(np.int32)
+    wh = rng.standard_normal((n, heads * f)).astype(np.float32)
+    src = rng.standard_normal((n, heads)).astype(np.float32)
+    dst = (3 * rng.standard_normal((n, heads))).astype(np.float32)
+    da = tg.DeviceCSR.from_numpy(n, n, rp, ci, np.ones(ci.size, np.float32))
+    plan = _plan(da, heads * f)
+    plan.set_precision(tg.PRECISION_FAST)
+    got = tg.gat_aggregate(plan, da, _t(gpu, wh), heads, f, _t(gpu, src),
+                           _t(gpu, dst)).cpu().numpy()
+    assert np.isfinite(got).all()
+    _check_gat_rows(got, np.concatenate([longs, rng.choice(n, size=400)]), rp, ci, wh, src, dst,
+                    heads, f)

@@ -597,9 +597,21 @@ __global__ __launch_bounds__(256) void gat_average_kernel(const float* __restric
     out[i * ldo + j] = finish_val(s, nullptr, 0, TG_ACT_NONE, post, exact != 0);
 }
 
-// Whether chunks take a wavefront each (gat_chunk_kernel, WAVE): as far as
-// measured (there), it was the faster at every size.
-inline bool gat_wave(int64_t n_chunks, int lpr) { return lpr < kWave && n_chunks <= 131072; }
+// Whether chunks take a wavefront each (gat_chunk_kernel, WAVE): a lane group's
+// time is the longest chunk's round trips, a wavefront's the number of chunks,
+// so the line is where the longest chunk is long for that number, or rows are
+// long on average.  Groups / wavefronts, us, 8 heads x 8 and 1 x 7 (power-law
+// rows unless noted): 131,000 rows, longest 1,024: 166 / 104, 160 / 90;
+// 131,000 rows of 3 entries each 35 / 95, 19 / 85; 32,000 of 3 each 16 / 29,
+// 12 / 26; 32,000 of 40 each 44 / 44, 23 / 26; 131,000 of 100 each 592 / 576,
+// 159 / 145, of 64 386 / 379, 103 / 94 (but 1 x 3 82 / 94).  Up to 8,192
+// chunks either runs in the time of the call, 13 on the host.
+inline bool gat_wave(const tg_spmm_plan_s& p, int lpr) {
+    const int64_t longest = p.n_split > 0 ? p.chunk : p.top;
+    return lpr < kWave && p.n_chunks <= 131072 &&
+           (p.n_chunks <= 8192 || p.n_chunks <= 128 * longest ||
+            p.nnz_bound >= 64 * p.n_chunks);
+}
 
 template <int VEC, int LPR, int VPL>
 void launch_gat(const tg_spmm_plan_s& p, const LaneLayout& L, GatArgs& a, hipStream_t s) {
@@ -615,7 +627,7 @@ void launch_gat(const tg_spmm_plan_s& p, const LaneLayout& L, GatArgs& a, hipStr
         return;
     }
     if (p.n_chunks > 0) {
-        const bool wave = gat_wave(p.n_chunks, LPR);
+        const bool wave = gat_wave(p, LPR);
         dim3 grid(static_cast<unsigned>(ceil_div(p.n_chunks, wave ? 256 / kWave : GPB)),
                   static_cast<unsigned>(L.n_tiles));
         if (wave)
