@@ -308,3 +308,34 @@ def test_gat_wave_lines(gpu, heads, f, n, long):
     assert np.isfinite(got).all()
     _check_gat_rows(got, np.concatenate([longs, rng.choice(n, size=400)]), rp, ci, wh, src, dst,
                     heads, f)
+
+
+@pytest.mark.parametrize("heads,f", [(1, 7), (8, 4), (1, 64)])
+@pytest.mark.parametrize("n,chunk", [(9000, 0), (9000, 16), (200, 0), (200, 16)])
+def test_gat_minus_inf_scores(gpu, heads, f, n, chunk):
+    """Scores of -inf weigh 0 wherever they stand in a row, one chunk or
+    several, in lane groups (9,000 short rows) and wavefronts alike; a row of
+    nothing else is NaN, as a softmax of it is."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(n + chunk + f)
+    lens = rng.integers(1, 4, size=n)
+    lens[:6] = [8, 9, 40, 40, 40, 0]
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = rng.integers(0, n - 1, size=rp[-1]).astype(np.int32)
+    ci[rp[0]:rp[0] + 7] = n - 1                        # all but the last entry
+    ci[rp[1]:rp[1] + 8] = n - 1                        # the first batch whole
+    ci[rp[2]:rp[2] + 32] = n - 1                       # whole chunks of 16
+    ci[rp[3] + 8:rp[3] + 40] = n - 1                   # after the others
+    ci[rp[4]:rp[5]] = n - 1                            # nothing else
+    wh = rng.standard_normal((n, heads * f)).astype(np.float32)
+    src = rng.standard_normal((n, heads)).astype(np.float32)
+    dst = (3 * rng.standard_normal((n, heads))).astype(np.float32)
+    dst[n - 1] = -np.inf
+    da = tg.DeviceCSR.from_numpy(n, n, rp, ci, np.ones(ci.size, np.float32))
+    plan = _plan(da, heads * f, chunk)
+    plan.set_precision(tg.PRECISION_FAST)
+    got = tg.gat_aggregate(plan, da, _t(gpu, wh), heads, f, _t(gpu, src),
+                           _t(gpu, dst)).cpu().numpy()
+    assert np.isnan(got[4]).all() and (got[5] == 0).all()
+    assert np.isfinite(np.delete(got, 4, axis=0)).all()
+    _check_gat_rows(got, [0, 1, 2, 3] + list(range(6, 100)), rp, ci, wh, src, dst, heads, f)

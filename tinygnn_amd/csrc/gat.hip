@@ -466,9 +466,9 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
                     ev[u][v] = lrelu(si[v] + ev[u][v], a.slope);
                     if (u < nv) mn = (mn < ev[u][v]) ? ev[u][v] : mn;
                 }
-                // a group that has met -inf scores only (another may hold
-                // the row's max) adds their exp(-inf) = 0
-                const float mx = WAVE && mn == -INFINITY ? 0.0f : mn;
+                // scores of -inf before any other (a later batch, or another
+                // group or chunk, may hold the row's max) add exp(-inf) = 0
+                const float mx = mn == -INFINITY ? 0.0f : mn;
                 const float sc = expf(m[v] - mx);
                 m[v] = mn;
                 s[v] *= sc;
@@ -507,19 +507,13 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
             }
         }
         if (part != 0) return;
-        // no score above -inf: exp(-inf - -inf), as one group's pass
-#pragma unroll
-        for (int v = 0; v < VPL; ++v)
-            if (m[v] == -INFINITY && b < e) {
-                s[v] = NAN;
-#pragma unroll
-                for (int k = 0; k < VEC; ++k) acc[v][k] = NAN;
-            }
     }
 
     if (split) {
         // the chunk's (max, sum) per head, written by the lane that owns the
-        // head's first feature
+        // head's first feature; (-inf, 0) where it has no other score: nothing,
+        // or NaN where no chunk of the row has (gat_reduce_kernel's exp(-inf -
+        // -inf))
         float* prow = a.partials + static_cast<int64_t>(ch.w) * a.ldp;
 #pragma unroll
         for (int v = 0; v < VPL; ++v) {
@@ -536,8 +530,9 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
         if (!ok[v]) continue;
-        // empty rows: s = 0 gives 0 before the bias (layers.cpp:1059)
-        const float inv = (s[v] > 0.0f) ? 1.0f / s[v] : 0.0f;
+        // empty rows: s = 0 gives 0 before the bias (layers.cpp:1059); a row
+        // of -inf scores alone is NaN, its max subtracted from itself
+        const float inv = m[v] == -INFINITY && b < e ? NAN : (s[v] > 0.0f) ? 1.0f / s[v] : 0.0f;
         gat_store<VEC>(a, row, fo[v], acc[v], inv);
     }
 }
