@@ -79,6 +79,37 @@ def test_edge_list_to_csr_partition_edges(gpu, restate, n, e, kind):
     np.testing.assert_array_equal(bits(v), bits(want.val))
 
 
+@pytest.mark.parametrize("n,rows", [
+    (65536, [0]), (65536, [65535]), (60000, [30000] * 100), (5000, [0, 64, 128, 4999]),
+    (5000, [64, 129, 4936]), (5000, [63, 128, 193, 4935]), ((1 << 22), [7, 1 << 20, (1 << 22) - 1]),
+    (3000, [1500] * 40000),   # sorted through memory
+])
+def test_edge_list_to_csr_empty_rows(gpu, restate, n, rows):
+    """Runs of empty rows of any length, 64 and 65 among them, between the
+    rows of a few edges."""
+    import tinygnn_amd as tg
+    src = np.array(rows, np.int32)
+    dst = np.random.default_rng(n).integers(0, n, size=src.size).astype(np.int32)
+    want = restate.edge_list_to_csr(src, dst, n)
+    rp, ci, v = tg.edge_list_to_csr(*_edges(gpu, src, dst), n).to_numpy()
+    np.testing.assert_array_equal(rp, want.row_ptr)
+    np.testing.assert_array_equal(ci, want.col_ind)
+    np.testing.assert_array_equal(bits(v), bits(want.val))
+
+
+@pytest.mark.parametrize("e", [1023, 1024, 1025, 262143, 262144, 262145])
+def test_edge_list_to_csr_shares(gpu, restate, e):
+    """The partition's shares of 1,024 edges, and whole tiles past 262,144."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(e)
+    src = np.sort(rng.integers(0, 9000, size=e)).astype(np.int32)
+    dst = rng.integers(0, 9000, size=e).astype(np.int32)
+    want = restate.edge_list_to_csr(src, dst, 9000)
+    rp, ci, v = tg.edge_list_to_csr(*_edges(gpu, src, dst), 9000).to_numpy()
+    np.testing.assert_array_equal(rp, want.row_ptr)
+    np.testing.assert_array_equal(ci, want.col_ind)
+
+
 def test_edge_list_to_csr_duplicates_and_self_edges(gpu, restate):
     import tinygnn_amd as tg
     rng = np.random.default_rng(9)

@@ -29,6 +29,7 @@ constexpr int kTileItems = 16;
 constexpr int kTile = kBlock * kTileItems;  // edges per partition step
 constexpr int kGrid = 256;                  // partition workgroups: one per CU (130 KB of LDS)
 constexpr int kEdgesPerBin = 4096;
+constexpr int kRowsPerBin = 2048;           // where rows are few edges each
 // Keys per thread that a workgroup sorts in LDS: 16 leave room for two
 // workgroups on a CU (80 KB of LDS, 64 registers), 32 fill one (144 KB).
 constexpr int kSortItems = 16, kSortItemsLong = 32;
@@ -44,7 +45,7 @@ constexpr uint32_t kOneF = 0x3f800000u;  // 1.0f
 static_assert(kLowBits <= 12 && (1 << kDigitBits) * kWaves == kBinsMax, "counter arrays");
 
 struct Build {
-    int64_t n, e, chunk;  // chunk: edges per partition workgroup, whole tiles
+    int64_t n, e, chunk;  // chunk: edges per partition workgroup
     int32_t bins, grid;
     int shift, dst_bits;
     const int32_t* src;
@@ -225,10 +226,30 @@ __device__ __forceinline__ int count_digit(int* counters, uint32_t d, bool valid
     return r;
 }
 
-// row_ptr of the rows that start at sorted position j (after row `prev`).
-__device__ __forceinline__ void start_rows(int32_t* row_ptr, int64_t row0, int prev, int row,
-                                           int32_t pos) {
-    for (int r = prev + 1; r <= row; ++r) row_ptr[row0 + r] = pos;
+// row_ptr of the rows that start at sorted position pos (after row `prev`), up
+// to kGap of them; where more are empty in a row, *wide says that every row is
+// to be searched for (search_rows), so that a row's cost does not depend on its
+// neighbours: 65,536 rows with one edge took 1.7 ms, now 0.08.  (Searches alone
+// took 98 us for 1M rows of one edge each, 92 so.)
+constexpr int kGap = 64;
+__device__ __forceinline__ void start_rows(int32_t* row_ptr, int prev, int row, int32_t pos,
+                                           int* wide) {
+    if (row - prev > kGap) *wide = 1;
+    for (int r = prev + 1; r <= min(row, prev + kGap); ++r) row_ptr[r] = pos;
+}
+
+__device__ __forceinline__ void search_rows(int32_t* row_ptr, int rows, const uint32_t* sorted,
+                                            int size, int dst_bits, int32_t base) {
+    for (int r = threadIdx.x; r < rows; r += kBlock) {
+        const uint32_t key = static_cast<uint32_t>(r) << dst_bits;
+        int lo = 0, hi = size;  // the first key not below it
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (sorted[mid] < key) lo = mid + 1;
+            else hi = mid;
+        }
+        row_ptr[r] = base + lo;
+    }
 }
 
 // One workgroup sorts one bucket (ITEMS = kSortItems: the short ones; else the
@@ -251,9 +272,11 @@ __global__ __launch_bounds__(kBlock, ITEMS == kSortItems ? 8 : 4) void bucket_so
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     const int key_bits = b.shift + b.dst_bits;
     const uint32_t dst_mask = (1u << b.dst_bits) - 1;
+    int* wide = cnt;  // (the counters are done with by then)
     if (bin == b.bins - 1 && threadIdx.x == 0) row_ptr[b.n] = static_cast<int32_t>(b.e);
+    row_ptr += row0;
     if (size == 0) {
-        for (int r = threadIdx.x; r < rows; r += kBlock) row_ptr[row0 + r] = base;
+        for (int r = threadIdx.x; r < rows; r += kBlock) row_ptr[r] = base;
         return;
     }
     if (ITEMS == kSortItems && size > ITEMS * kBlock) return;  // listed
@@ -334,15 +357,19 @@ __global__ __launch_bounds__(kBlock, ITEMS == kSortItems ? 8 : 4) void bucket_so
                 for (int i = 0; i < ITEMS; ++i) k[i] = buf[first + i * kWave];  // within buf
             }
         }
+        if (threadIdx.x == 0) *wide = 0;
+        __syncthreads();
         for (int j = threadIdx.x; j < size; j += kBlock) {
             const uint32_t x = buf[j];
             const int row = static_cast<int>(x >> b.dst_bits);
             const int prev = j > 0 ? static_cast<int>(buf[j - 1] >> b.dst_bits) : -1;
             other[j] = x & dst_mask;
             in[j] = kOneF;
-            start_rows(row_ptr, row0, prev, row, base + j);
-            if (j == size - 1) start_rows(row_ptr, row0, row, rows - 1, base + size);
+            start_rows(row_ptr, prev, row, base + j, wide);
+            if (j == size - 1) start_rows(row_ptr, row, rows - 1, base + size, wide);
         }
+        __syncthreads();
+        if (*wide) search_rows(row_ptr, rows, buf, size, b.dst_bits, base);
         return;
     }
     if constexpr (ITEMS == kSortItems) return;
@@ -393,12 +420,16 @@ __global__ __launch_bounds__(kBlock, ITEMS == kSortItems ? 8 : 4) void bucket_so
         in = other;
         other = t;
     }
+    if (threadIdx.x == 0) *wide = 0;
+    __syncthreads();
     for (int j = threadIdx.x; j < size; j += kBlock) {
         const int row = static_cast<int>(in[j] >> b.dst_bits);
         const int prev = j > 0 ? static_cast<int>(in[j - 1] >> b.dst_bits) : -1;
-        start_rows(row_ptr, row0, prev, row, base + j);
-        if (j == size - 1) start_rows(row_ptr, row0, row, rows - 1, base + size);
+        start_rows(row_ptr, prev, row, base + j, wide);
+        if (j == size - 1) start_rows(row_ptr, row, rows - 1, base + size, wide);
     }
+    __syncthreads();
+    if (*wide) search_rows(row_ptr, rows, in, size, b.dst_bits, base);
     __syncthreads();
     for (int j = threadIdx.x; j < size; j += kBlock) {
         const uint32_t x = in[j];
@@ -418,13 +449,15 @@ Build shape(int64_t n, int64_t e) {
     b.n = n;
     b.e = e;
     b.dst_bits = bits_for(n);
-    const int64_t want = std::clamp<int64_t>(e / kEdgesPerBin, 1, kBinsMax);
+    const int64_t want =
+        std::clamp<int64_t>(std::max(e / kEdgesPerBin, n / kRowsPerBin), 1, kBinsMax);
     while (b.shift < 32 - b.dst_bits && ceil_div(n, int64_t(1) << b.shift) > want) ++b.shift;
     b.bins = static_cast<int32_t>(ceil_div(n, int64_t(1) << b.shift));
-    const int64_t tiles = ceil_div(e, kTile);
-    const int64_t per = ceil_div(tiles, kGrid);
-    b.chunk = per * kTile;
-    b.grid = static_cast<int32_t>(ceil_div(tiles, per));
+    // few edges: shares of 1,024, since equal sources contend for an LDS counter
+    // (20,000 edges ordered by source 108 us in whole tiles, 80 in shares,
+    // 87 by the general build)
+    b.chunk = e <= kGrid * kBlock ? kBlock : ceil_div(ceil_div(e, kTile), kGrid) * kTile;
+    b.grid = static_cast<int32_t>(ceil_div(e, b.chunk));
     return b;
 }
 
