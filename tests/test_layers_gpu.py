@@ -72,6 +72,24 @@ def test_sage_dual_tiles_bitexact(gpu, restate, n, f_out, f_in):
     np.testing.assert_array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("f_in", [3, 17, 24, 31])
+def test_sage_dual_short_k_bitexact(gpu, restate, f_in):
+    """The dual product's tiles of 16 k slots, wide outputs (133: the tail's
+    five columns aside), bit for bit."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(f_in)
+    n, f_out = 8300, 133
+    a = random_csr(rng, n, n, avg_deg=2, max_deg=9, empty_frac=0.1)
+    h = rng.standard_normal((n, f_in)).astype(np.float32)
+    wn = rng.standard_normal((f_in, f_out)).astype(np.float32)
+    ws = rng.standard_normal((f_in, f_out)).astype(np.float32)
+    want = restate.sage_layer(a, h, wn, ws, None, act=0, agg=1)
+    da = _dev(a)
+    got = tg.sage_forward(_plan(da, f_out), da, _t(gpu, h), _t(gpu, wn), _t(gpu, ws), None,
+                          act=0, agg=1, dataflow=tg.SAGE_CONCAT).cpu().numpy()
+    np.testing.assert_array_equal(bits(got), bits(want))
+
+
 @pytest.mark.parametrize("agg", [0, 1])
 def test_sage_aggregate_split_rows(gpu, restate, agg):
     import tinygnn_amd as tg

@@ -879,12 +879,16 @@ void launch_chain_kt(const GemmArgs& g, hipStream_t s) {
 // larger ones take tiles that read B less often.  Either side of each line,
 // us: n = 16: 20,000 x 500 12.5 / 16.4, 60,000 x 300 19.8 / 18.8; n <= 32:
 // 2,708 x 1,433 x 32 17.7 / 32.1, 30,000 x 700 x 24 32.4 / 26.4; n > 32:
-// 12,000 x 300 x 60 13.3 / 15.2, 20,000 x 300 x 60 22.0 / 21.1; k < 32, where
-// a 32-slot tile is mostly padding: 400,000 x 8 x 200 140 against 176.
+// 12,000 x 300 x 60 13.3 / 15.2, 20,000 x 300 x 60 22.0 / 21.1.  16 slots of k
+// where a tile of 32 would be mostly padding, 16 / 32: 400,000 x 8 x 200 140 /
+// 176, 500,000 x 8 x 7 12.4 / 20.4, 500,000 x 31 x 16 20.9 / 24.2, 100,000 x 33 x
+// 100 27 / 33, 500,000 x 33 x 200 241 / 288.
 template <bool DUAL>
 void launch_chain(const GemmArgs& g, hipStream_t s) {
+    const int64_t slots = g.k1 * (DUAL ? 2 : 1);
     if (g.n <= 16) {
         if (g.m <= 32768) return launch_chain_kt<1, 1, 1, 1, 64, DUAL>(g, s);
+        if (slots < 32) return launch_chain_kt<2, 1, 4, 1, 16, DUAL>(g, s);
         return launch_chain_kt<2, 1, 4, 1, 32, DUAL>(g, s);
     }
     if (g.n <= 32) {
@@ -892,7 +896,8 @@ void launch_chain(const GemmArgs& g, hipStream_t s) {
         return launch_chain_kt<1, 2, 4, 1, 32, DUAL>(g, s);
     }
     if (g.m * ceil_div(g.n, 64) <= 16384) return launch_chain_kt<1, 1, 1, 4, 64, DUAL>(g, s);
-    if (g.k1 * (DUAL ? 2 : 1) < 32) return launch_chain_kt<2, 2, 2, 2, 16, DUAL>(g, s);
+    if (slots < 32 || (slots < 64 && (slots - 1) % 32 < 16))
+        return launch_chain_kt<2, 2, 2, 2, 16, DUAL>(g, s);
     launch_chain_as<2, 2, 2, 2, 32, DUAL, true>(g, s);
 }
 
