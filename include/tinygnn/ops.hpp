@@ -9,9 +9,9 @@
 
 namespace tinygnn {
 
-/// C = A * B, both Dense (ops.cpp:70-162).  Small products are bit-identical
-/// to the reference; wide ones (n >= 64, k >= 32, m*n*k >= 2^32) run on fp32
-/// MFMA (within 1e-4 relative).
+/// C = A * B, both Dense (ops.cpp:70-162).  Bit-identical to the reference,
+/// but for large products (k >= 32 and n >= 64, m*n*k >= 2^32 or n < 64, m*k >=
+/// 2^25), whose fp32 sums may run in another order (within 1e-4 relative).
 Tensor matmul(const Tensor& A, const Tensor& B);
 
 /// C = A * B, A SparseCSR, B Dense (ops.cpp:198-297).  Every row is one

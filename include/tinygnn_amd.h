@@ -221,8 +221,9 @@ int tg_spmm_noalloc(int64_t m, int64_t k, int64_t f, int64_t nnz, const int32_t*
  * epilogue (bias add, then activation) that equals calling add_bias
  * (ops.cpp:622) and relu_inplace / elu_inplace afterwards.
  * algo: TG_GEMM_AUTO may regroup the sums of large products (n >= 64, k >= 32
- * and m*n*k >= 2^32; n < 64, k >= 32 and m*k >= 2^25), else in order; TG_GEMM_INORDER is bit-identical
- * to the reference (one fma chain over k ascending from 0 per output);
+ * and m*n*k >= 2^32; n < 64, k >= 32 and m*k >= 2^25), and sums others in
+ * order; TG_GEMM_INORDER is bit-identical to the reference (one fma chain over
+ * k ascending from 0 per output);
  * TG_GEMM_MFMA uses v_mfma_f32_16x16x4f32 (regrouped sums: within
  * tolerance, not bit-identical).
  * ------------------------------------------------------------------------ */

@@ -75,6 +75,26 @@ def test_matmul_mfma_bound(gpu, m, k, n):
     assert (np.abs(got - exact) <= bound).all(), float((np.abs(got - exact) / bound).max())
 
 
+@pytest.mark.parametrize("m,k,n,chain", [
+    (132000, 512, 64, True), (130000, 258, 130, True), (185000, 192, 121, True),
+    (186000, 191, 121, False), (561000, 64, 121, False), (100000, 512, 128, True),
+    (30000, 700, 256, False), (100000, 672, 128, False)])
+def test_matmul_auto_lines(gpu, m, k, n, chain):
+    """Where AUTO may regroup the sums: the in-order product's bits where it
+    takes that kernel, the fp32 bound around them elsewhere."""
+    import tinygnn_amd as tg
+    torch = gpu
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n)
+    a = torch.randn(m, k, generator=g, device="cuda")
+    b = torch.randn(k, n, generator=g, device="cuda")
+    got, order = tg.matmul(a, b), tg.matmul(a, b, algo=tg.GEMM_INORDER)
+    assert torch.equal(got, order) == chain
+    # either sum is within (k + 2) 2^-24 of the exact one; |a| |b| in fp32 is too
+    bound = 2.1 * (k + 2) * 2.0 ** -24 * torch.mm(a.abs(), b.abs())
+    assert bool(((got - order).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("n", [96, 41])
 @pytest.mark.parametrize("algo", [1, 2])
 @pytest.mark.parametrize("epi", [0, 1, 2])

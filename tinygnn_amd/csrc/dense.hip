@@ -960,12 +960,10 @@ void softmax_launch(bool log, int64_t rows, int64_t cols, float* x, hipStream_t 
 }  // namespace
 
 int resolve_gemm_algo(int algo, int64_t m, int64_t n, int64_t k) {
-    // MFMA only where the product is a real contraction (wide n, deep k and
-    // enough work to fill the chip); small products keep the bit-exact
-    // in-order kernel.
-    // A thin product (n < 64) takes MFMA when A alone is large (m k >= 2^25:
-    // config E's n x 256 x 41 layer-2 transforms, 212 us in order); Cora-scale
-    // products stay in order.
+    // AUTO may regroup the sums (TG_GEMM_MFMA here; which kernel then runs:
+    // chain_tiles) only where the product is a real contraction, with enough
+    // work to fill the chip: wide n and deep k, or for a thin product (n < 64)
+    // A alone large (m k >= 2^25); others stay bit-exact.
     if (algo == TG_GEMM_AUTO) {
         if (n >= 64) return (k >= 32 && m * n * k >= (int64_t(1) << 32)) ? TG_GEMM_MFMA
                                                                           : TG_GEMM_INORDER;
@@ -974,12 +972,24 @@ int resolve_gemm_algo(int algo, int64_t m, int64_t n, int64_t k) {
     return algo;
 }
 
-// Where AUTO may regroup the k order, the 128 x 128 tiles of gemm_mfma_kernel
-// pay from this many products on; below, their last wave leaves most of the
-// chip idle and the smaller tiles of gemm_chain_kernel are faster: 100,000 x
-// 512 x 128 (2^32.6) 139 against 155 us, 100,003 x 257 x 121 91 / 115, but
-// 500,000 x 256 x 256 (2^34.9) 692 / 616 and 232,965 x 602 x 256 697 / 645.
-constexpr int64_t kMfmaTilesOps = int64_t(1) << 33;
+// Where AUTO may regroup the k order, whether the 64 x 64 tiles of
+// gemm_chain_kernel are faster than the 128 x 128 of gemm_mfma_kernel.  Per
+// padded output the larger tiles are the faster by a sixth, more where k is
+// short, so they lose where they pad more columns, where a partial last column
+// tile's guarded loads count (k long), or where their last round over the 256
+// compute units is mostly empty.  Large / small tiles, us: 244,589 x 512 x 64 235
+// / 171, 34,945 x 1,433 x 130 319 / 202; 105,080 x 512 x 121 202 / 141, 57,247 x 700
+// x 200 275 / 201, but 1,034,955 x 64 x 121 310 / 342; 100,000 x 512 x 128 (3.05
+// rounds) 155 / 139, but 30,000 x 700 x 256 (1.84) 108 / 117 and 120,000 x 100 x
+// 512 (14.7) 173 / 207.  From 2^33 on the large ones: 500,000 x 256 x 256 616 /
+// 692, 232,965 x 602 x 256 645 / 697.
+bool chain_tiles(int64_t m, int64_t n, int64_t k) {
+    if (n < 64 || m * n * k >= int64_t(1) << 33) return false;
+    const int64_t last = n % 128;
+    if (last > 0) return last <= 64 || k >= 192;
+    const int64_t tiles = ceil_div(m, 128) * (n / 128);
+    return 4 * 256 * ceil_div(tiles, 256) > 5 * tiles;
+}
 
 void gemm(const GemmArgs& g, int algo, hipStream_t s) {
     require(g.m >= 0 && g.n >= 0 && g.k1 >= 0 && g.k2 >= 0, "matmul: negative dimension");
@@ -997,11 +1007,10 @@ void gemm(const GemmArgs& g, int algo, hipStream_t s) {
     const bool dual = g.a2 != nullptr;
     if (dual)
         require(g.b2 && g.lda2 >= g.k2 && g.ldb2 >= g.n, "matmul: bad second operand pair");
-    const int64_t ops = g.m * g.n * (g.k1 + g.k2);
     const bool chain_fits = !dual || g.k1 == g.k2;
     const bool any_order = algo == TG_GEMM_AUTO;
     algo = resolve_gemm_algo(algo, g.m, g.n, g.k1 + g.k2);
-    if (any_order && algo == TG_GEMM_MFMA && g.n >= 64 && chain_fits && ops < kMfmaTilesOps) {
+    if (any_order && algo == TG_GEMM_MFMA && chain_fits && chain_tiles(g.m, g.n, g.k1 + g.k2)) {
         if (!dual) return launch_chain<false>(g, s);
         return launch_chain<true>(g, s);  // as one chain, without scalar-tail columns
     }
