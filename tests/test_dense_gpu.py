@@ -58,6 +58,63 @@ def test_matmul_chain_tiles(gpu, restate, m, n, k):
     np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
 
 
+def _range_operands(m, k, n, seed):
+    """Operands whose products and sums leave the normal range: denormal inputs
+    and products, sums that overflow midway, and cancellations that show the
+    order of the sum."""
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    a[1::5] *= np.float32(1e-20)
+    a[2::5] *= np.float32(1e-40)   # denormal
+    a[3::5] *= np.float32(1e19)
+    a[4::5, ::3] *= np.float32(1e8)
+    a[4::5, 2::3] = -a[4::5, : k - 2: 3]
+    b[:, 1::4] *= np.float32(1e-20)
+    b[:, 2::4] *= np.float32(1e19)
+    b[2::3, 3::4] = b[: k - 2: 3, 3::4]
+    return a, b
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 70, 16), (8200, 65, 32), (205, 129, 48), (40000, 35, 15),
+                                   (40000, 17, 7), (8300, 40, 65), (8300, 64, 70)])
+def test_matmul_chain_range(gpu, restate, m, k, n):
+    """The in-order product over denormals, overflow midway and cancellation,
+    in every tile, bit for bit against the CPU's fma chain."""
+    import tinygnn_amd as tg
+    a, b = _range_operands(m, k, n, m + k + n)
+    want = restate.matmul(a, b)
+    tiny = (np.abs(want) > 0) & (np.abs(want) < np.finfo(np.float32).tiny)
+    assert tiny.any() and np.isinf(want).any()
+    got = tg.matmul(_t(gpu, a), _t(gpu, b), algo=tg.GEMM_INORDER).cpu().numpy()
+    nan = np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 70, 16), (8200, 35, 31), (8300, 20, 77)])
+def test_sage_dual_range(gpu, restate, m, k, n):
+    """The dual product's chain and tail columns over the same operands, both
+    pairs: every row's one neighbour has its own row's kind (max, so the
+    aggregate is a copy)."""
+    import oracle
+    import tinygnn_amd as tg
+    h, wn = _range_operands(m, k, n, m + k)
+    ws = _range_operands(m, k, n, m + k + 1)[1]
+    rp = np.arange(m + 1, dtype=np.int32)
+    g = oracle.CSR(m, m, rp, ((rp[:-1] + 5) % m).astype(np.int32), np.ones(m, np.float32))
+    want = restate.sage_layer(g, h, wn, ws, None, act=0, agg=1)
+    tiny = (np.abs(want) > 0) & (np.abs(want) < np.finfo(np.float32).tiny)
+    assert tiny.any() and np.isinf(want).any()
+    d = tg.DeviceCSR.from_numpy(m, m, g.row_ptr, g.col_ind, g.val)
+    got = tg.sage_forward(tg.SpmmPlan(d.row_ptr, m, m, max(k, n)), d, _t(gpu, h), _t(gpu, wn),
+                          _t(gpu, ws), None, act=0, agg=1,
+                          dataflow=tg.SAGE_CONCAT).cpu().numpy()
+    nan = np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
 @pytest.mark.parametrize("m,k,n", [(128, 16, 128), (1000, 602, 256), (777, 256, 41),
                                    (300, 33, 130), (64, 1433, 64),
                                    # thin products (n <= 64: 16-column MFMA tiles), k not a
