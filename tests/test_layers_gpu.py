@@ -127,13 +127,15 @@ def test_sage_transform_first(gpu, restate, f_in, f_out):
     assert_close(got, want, what="sage transform-first")
 
 
-def test_sage_concat_mfma_dual(gpu, restate):
-    """Concat dataflow large enough for the MFMA GEMM (m*n*k >= 2^32): the
-    dual product [AGG | H] x [Wn ; Ws] runs as two K segments of one MFMA
-    kernel; within tolerance of the reference."""
+@pytest.mark.parametrize("n", [40000, 90000])
+def test_sage_concat_mfma_dual(gpu, restate, n):
+    """Concat dataflow large enough to regroup the sums of the dual product
+    [AGG | H] x [Wn ; Ws]: from 2^33 multiply-adds on (90,000 rows) as two K
+    segments of gemm_mfma_kernel, below as one chain without scalar-tail
+    columns; within tolerance of the reference."""
     import tinygnn_amd as tg
     rng = np.random.default_rng(21)
-    n, f_in, f_out = 40000, 256, 210
+    f_in, f_out = 256, 210
     a = random_csr(rng, n, n, avg_deg=3, max_deg=50, empty_frac=0.05)
     h = rng.standard_normal((n, f_in)).astype(np.float32)
     s = np.float32(1.0 / np.sqrt(f_in))
