@@ -25,8 +25,8 @@ def _edges(gpu, src, dst):
 
 @pytest.mark.parametrize("n,e,dmax,seed", [
     (1, 0, 1, 0), (5, 1, 1, 1), (300, 4000, 64, 2), (2000, 60000, 900, 3),
-    (500, 120000, 40000, 4),     # rows > 16384: the global bitonic path
-    (64, 200000, 100000, 5),     # padded length 131072: several global stages
+    (500, 120000, 40000, 4),     # a bucket over 32,768: sorted through memory
+    (64, 200000, 100000, 5),
 ])
 def test_edge_list_to_csr_bitexact(gpu, restate, n, e, dmax, seed):
     import tinygnn_amd as tg
@@ -72,6 +72,30 @@ def test_edge_list_to_csr_partition_edges(gpu, restate, n, e, kind):
         rng.shuffle(src)
     dst = rng.integers(0, n, size=e).astype(np.int32)
     dst[:: 7] = n - 1
+    want = restate.edge_list_to_csr(src, dst, n)
+    rp, ci, v = tg.edge_list_to_csr(*_edges(gpu, src, dst), n).to_numpy()
+    np.testing.assert_array_equal(rp, want.row_ptr)
+    np.testing.assert_array_equal(ci, want.col_ind)
+    np.testing.assert_array_equal(bits(v), bits(want.val))
+
+
+@pytest.mark.parametrize("lens", [
+    [270000], [65, 100, 1023, 1024, 270000, 64, 2, 1],     # with every length class
+    [1025, 2000, 16383, 16384, 300000, 1024, 0, 63],
+    [16385, 17000, 270000, 40000, 0, 131073, 70, 1500],    # several long rows: segments, stages
+])
+def test_edge_list_to_csr_general_rows(gpu, restate, lens):
+    """The general build, which a bucket of more than 262,144 edges takes: its
+    sorts of rows up to 64, 1,024 and 16,384 entries and of several longer
+    ones, beside 500 rows of a few edges."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(len(lens) + lens[0])
+    n = 600
+    deg = rng.integers(0, 70, size=n)
+    deg[rng.choice(n, size=len(lens), replace=False)] = lens
+    src = np.repeat(np.arange(n), deg).astype(np.int32)
+    rng.shuffle(src)
+    dst = rng.integers(0, n, size=src.size).astype(np.int32)
     want = restate.edge_list_to_csr(src, dst, n)
     rp, ci, v = tg.edge_list_to_csr(*_edges(gpu, src, dst), n).to_numpy()
     np.testing.assert_array_equal(rp, want.row_ptr)
