@@ -42,11 +42,10 @@ def _finish(stream) -> None:
     call are torch's memory of the current stream: reading a result's size, the
     caller's next operation and the allocator's reuse of what the caller drops
     are all ordered there, not after another stream's kernels."""
-    torch = _torch()
-    if stream is None or int(stream.cuda_stream) == int(torch.cuda.current_stream().cuda_stream):
+    if stream is None or int(stream.cuda_stream) == stream_handle():
         return
     wait = getattr(stream, "synchronize", None)
-    (wait or torch.cuda.ExternalStream(int(stream.cuda_stream)).synchronize)()
+    (wait or _torch().cuda.ExternalStream(int(stream.cuda_stream)).synchronize)()
 
 
 def trim() -> None:
