@@ -70,13 +70,10 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
     if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(&hist[kTopSlot], top);
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * kPlanBins; i += blockDim.x) {
-        if (i == kTopSlot) {  // (few of the workgroups raise it)
-            if (hist[i] > __hip_atomic_load(&bin_count[i], __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT))
-                atomicMax(&bin_count[i], hist[i]);
-        } else if (hist[i]) {
+        if (i == kTopSlot)
+            atomicMax(&bin_count[i], hist[i]);
+        else if (hist[i])
             atomicAdd(&bin_count[i], hist[i]);
-        }
     }
 }
 
