@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void gat_average_kernel(const float* __restric
 // chunks either runs in the time of the call, 13 on the host.
 inline bool gat_wave(const tg_spmm_plan_s& p, int lpr) {
     const int64_t longest = p.n_split > 0 ? p.chunk : p.top;
-    return lpr < kWave && p.n_chunks <= 131072 &&
+    return lpr < kWave && p.n_chunks <= kTopRows &&
            (p.n_chunks <= 8192 || p.n_chunks <= 128 * longest ||
             p.nnz_bound >= 64 * p.n_chunks);
 }

@@ -65,14 +65,17 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
             atomicAdd(&hist[kPlanBins + chunk_bin(deg)], 1);
         }
     }
+    if (m <= kTopRows) {
 #pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d, kWave));
-    if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(&hist[kTopSlot], top);
+        for (int d = kWave / 2; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d, kWave));
+        if ((threadIdx.x & (kWave - 1)) == 0 && top > 0) atomicMax(&hist[kTopSlot], top);
+    }
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * kPlanBins; i += blockDim.x) {
+        if (hist[i] == 0) continue;
         if (i == kTopSlot)
             atomicMax(&bin_count[i], hist[i]);
-        else if (hist[i])
+        else
             atomicAdd(&bin_count[i], hist[i]);
     }
 }
