@@ -181,6 +181,16 @@ def test_short_field_paths(gpu, restate, offset):
             assert _gpu_feats(gpu, t, offset=offset) == _ora_feats(restate, t), (total, tail)
 
 
+def test_exponent_fields(gpu, restate):
+    """Fields in exponent form, at every alignment in the parser's window, and
+    the letter in their place in fields that are no numbers."""
+    for f in ("1.5e-03", "2e+10", "1E-05", "-1.23456789e+02", "e-05", "1e-45", "1.5f-03", "12e4",
+              "1e400", "0e+00"):
+        for pad in range(4):
+            t = ("0," + "7" * pad + "1," + f + ",2.5\n1,1,1.25," + f + "\n").encode()
+            assert _gpu_feats(gpu, t) == _ora_feats(restate, t), (f, pad)
+
+
 def test_large_files(gpu, restate, tmp_path):
     """Millions of edge lines and a 30,000 x 100 feature table through the
     file path (pinned staging, overlapped copies), then a planted defect near
