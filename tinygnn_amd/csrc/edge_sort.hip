@@ -8,9 +8,9 @@
 // (src and dst twice, the keys once each way, the outputs once), except the
 // partition's writes, runs of a tile's edges of one bucket; the sorts are bound
 // by the vector instructions that rank the keys (about 270 per 64 keys).
-// 1M nodes, 50M edges in random order: 1.23 ms (count 0.12, partition 0.27,
+// 1M nodes, 50M edges in random order: 1.16 ms (count 0.12, partition 0.27,
 // sorts 0.71).  The general build in graph.hip, which counts and places edges
-// by one device atomic each and sorts row by row, takes 8.0 ms (2.5 count, 2.7
+// by one device atomic each and sorts row by row, takes 7.8 ms (2.5 count, 2.7
 // place, 2.1 sorts).  8,192 buckets: partition 0.38, sorts 0.75 ms; one sort
 // kernel for all buckets at one workgroup per CU: 0.91 ms.
 #include "common.hpp"
@@ -229,8 +229,8 @@ __device__ __forceinline__ int count_digit(int* counters, uint32_t d, bool valid
 // row_ptr of the rows that start at sorted position pos (after row `prev`), up
 // to kGap of them; where more are empty in a row, *wide says that every row is
 // to be searched for (search_rows), so that a row's cost does not depend on its
-// neighbours: 65,536 rows with one edge took 1.7 ms, now 0.08.  (Searches alone
-// took 98 us for 1M rows of one edge each, 92 so.)
+// neighbours: 65,536 rows, 131 edges in one of them, took 1.7 ms, now 0.07.
+// (Searches alone took 98 us for 1M rows of one edge on average, 92 so.)
 constexpr int kGap = 64;
 __device__ __forceinline__ void start_rows(int32_t* row_ptr, int prev, int row, int32_t pos,
                                            int* wide) {
