@@ -359,3 +359,47 @@ def test_gat_minus_inf_scores(gpu, heads, f, n, chunk):
     assert np.isnan(got[4]).all() and (got[5] == 0).all()
     assert np.isfinite(np.delete(got, 4, axis=0)).all()
     _check_gat_rows(got, [0, 1, 2, 3] + list(range(6, 100)), rp, ci, wh, src, dst, heads, f)
+
+
+@pytest.mark.parametrize("long", [0, 900])
+@pytest.mark.parametrize("heads,f,concat", [(2, 8, True), (4, 16, False), (8, 3, False),
+                                            (1, 33, True)])
+def test_gat_forms(gpu, heads, f, concat, long):
+    """Lane groups (9,000 short rows) and wavefronts (one of 900 beside them)
+    over the forms that calls take: Wh as a view of a wider matrix, bias, ELU,
+    averaged heads and empty rows, against fp64."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(heads * f + long)
+    n = 9000
+    lens = rng.integers(0, 4, size=n)
+    if long:
+        lens[17] = long
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = rng.integers(0, n, size=rp[-1]).astype(np.int32)
+    wh = rng.standard_normal((n, heads * f)).astype(np.float32)
+    src = rng.standard_normal((n, heads)).astype(np.float32)
+    dst = rng.standard_normal((n, heads)).astype(np.float32)
+    bias = rng.standard_normal(heads * f).astype(np.float32)
+    da = tg.DeviceCSR.from_numpy(n, n, rp, ci, np.ones(ci.size, np.float32))
+    plan = _plan(da, heads * f)
+    plan.set_precision(tg.PRECISION_FAST)
+    rows = [17] + list(range(60))
+    want = np.zeros((len(rows), heads, f))
+    for k, i in enumerate(rows):
+        c = ci[rp[i]:rp[i + 1]]
+        if len(c):
+            e = src[i].astype(np.float64) + dst[c].astype(np.float64)
+            p = np.exp(np.where(e >= 0, e, 0.2 * e))
+            w = wh[c].astype(np.float64).reshape(-1, heads, f)
+            want[k] = (p[:, :, None] * w).sum(0) / p.sum(0)[:, None]
+    want += bias.astype(np.float64).reshape(heads, f)
+    want = want.reshape(len(rows), -1) if concat else want.mean(axis=1)
+    want = np.where(want < 0, np.expm1(want), want)
+    for off, pad in ((0, 0), (3, 2), (4, 4)):
+        wide = gpu.zeros(n, heads * f + off + pad, device="cuda")
+        view = wide[:, off:off + heads * f]
+        view.copy_(_t(gpu, wh))
+        got = tg.gat_aggregate(plan, da, view, heads, f, _t(gpu, src), _t(gpu, dst),
+                               bias=_t(gpu, bias), post=tg.POST_ELU, concat=concat)
+        # (900 + 3 * 32 + 16) 2^-24 of a weighted mean of magnitudes near 1
+        assert_close(got.cpu().numpy()[rows], want, rtol=6.1e-5, atol=6.1e-5, what="gat forms")

@@ -90,6 +90,49 @@ def test_spmm_plan_shapes_bitexact(gpu, restate, n, row, long, f):
     np.testing.assert_array_equal(bits(got), bits(restate.spmm(a, b)))
 
 
+@pytest.mark.parametrize("long", [0, 900])
+@pytest.mark.parametrize("f", [2, 5, 16, 33, 64, 100, 128])
+def test_spmm_forms_bitexact(gpu, restate, f, long):
+    """Both kernels for a chunk (9,000 short rows: lane groups; with one of 900:
+    wavefronts) over the forms that calls take: B and the output as views of
+    wider matrices at any column, bias and activation, and the mean and max
+    aggregates, bit for bit; the views' other columns stay as they were."""
+    import tinygnn_amd as tg
+    rng = np.random.default_rng(f + long)
+    n = 9000
+    deg = rng.integers(0, 5, size=n)
+    if long:
+        deg[n // 2] = long
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    a = oracle.CSR(n, n, rp, rng.integers(0, n, rp[-1]).astype(np.int32),
+                   rng.standard_normal(rp[-1]).astype(np.float32))
+    b = rng.standard_normal((n, f)).astype(np.float32)
+    bias = rng.standard_normal(f).astype(np.float32)
+    da = tg.DeviceCSR.from_numpy(n, n, a.row_ptr, a.col_ind, a.val)
+    plan = tg.SpmmPlan(da.row_ptr, n, a.nnz, f)
+    want = restate.spmm(a, b)
+    act = restate.add_bias(want, bias)
+    act = np.where(act > 0, act, np.float32(0))
+    eye, zero = np.eye(f, dtype=np.float32), np.zeros((f, f), np.float32)
+    mean = restate.sage_layer(a, b, eye, zero, None, act=0, agg=0)
+    most = restate.sage_max_aggregate(a, b)
+    for off, pad in ((0, 0), (0, 3), (1, 4), (4, 4)):
+        wide = gpu.zeros(n, f + off + pad, device="cuda")
+        view = wide[:, off:off + f]
+        view.copy_(gpu.from_numpy(b))
+        outs = gpu.full((n, f + off + pad), 7.0, device="cuda")
+        out = outs[:, off:off + f]
+        tg.spmm(da, view, plan, out=out)
+        np.testing.assert_array_equal(bits(out.cpu().numpy()), bits(want))
+        tg.spmm_epilogue(da, view, plan, gpu.from_numpy(bias).cuda(), tg.EPI_RELU, out=out)
+        np.testing.assert_array_equal(out.cpu().numpy(), act)
+        rest = gpu.cat([outs[:, :off], outs[:, off + f:]], 1)
+        assert bool((rest == 7.0).all())
+        np.testing.assert_array_equal(tg.sage_aggregate(plan, da, view, 0).cpu().numpy(), mean)
+        np.testing.assert_array_equal(bits(tg.sage_aggregate(plan, da, view, 1).cpu().numpy()),
+                                      bits(most))
+
+
 @pytest.mark.parametrize("chunk", [1, 7, 64, 256])
 @pytest.mark.parametrize("f", [2, 3, 4, 41, 128, 512])
 def test_spmm_split_rows_exact(gpu, restate, f, chunk):

@@ -1718,10 +1718,10 @@ void launch_long(const PlanView& p, int tw, int64_t f, const int32_t* ci, const 
 // every column's chain is agg_chunk_kernel's, in nonzero order.  The LDS
 // regions belong to one wavefront each, so no barrier of the workgroup is
 // needed (their trip counts differ).
-// Against agg_chunk_kernel, weighted SpMM, same bits, us: 2,708 rows of 4
-// entries x 16 columns 18 -> 11, 3,000 of 100 x 16 31 -> 11, 1,000 of 250 x 64
-// 46 -> 25, 8,000 of 60 x 32 39 -> 17, 32,000 of 40 x 16 119 -> 59 (its rows
-// over 1,024 entries, in agg_long_kernel, included).
+// Against agg_chunk_kernel, weighted SpMM of power-law rows, same bits, us:
+// 2,708 rows of 4 entries on average x 16 columns 18 -> 11, 3,000 of 100 x 16 31
+// -> 11, 1,000 of 250 x 64 46 -> 25, 8,000 of 60 x 32 39 -> 17, 32,000 of 40 x 16
+// 119 -> 59 (its rows over 1,024 entries, in agg_long_kernel, included).
 template <int VEC, int TW, int MODE>
 __global__ __launch_bounds__(256) void agg_small_kernel(
     const int4* __restrict__ chunks, int64_t n_chunks, const int32_t* __restrict__ ci,
