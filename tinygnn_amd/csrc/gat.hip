@@ -414,12 +414,14 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
     // One pass with an online softmax per lane vector (its head): running
     // max m, running sum s of exp(e - m), and acc = sum exp(e - m) Wh_j; a
     // larger max rescales s and acc by exp(m_old - m_new) (exactly 1 when
-    // the max is unchanged, 0 from the initial -inf).  Lanes of one head see
-    // the same scores, so their (m, s) agree.
+    // the max is unchanged, 0 from the initial one).  It starts from the lowest
+    // finite value, so that scores of -inf add exp(-inf) = 0 wherever they
+    // stand; a chunk of nothing else ends with s = 0.  Lanes of one head see the
+    // same scores, so their (m, s) agree.
     float m[VPL], s[VPL], acc[VPL][VEC];
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
-        m[v] = -INFINITY;
+        m[v] = -__FLT_MAX__;
         s[v] = 0.0f;
 #pragma unroll
         for (int k = 0; k < VEC; ++k) acc[v][k] = 0.0f;
@@ -466,10 +468,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
                     ev[u][v] = lrelu(si[v] + ev[u][v], a.slope);
                     if (u < nv) mn = (mn < ev[u][v]) ? ev[u][v] : mn;
                 }
-                // scores of -inf before any other (a later batch, or another
-                // group or chunk, may hold the row's max) add exp(-inf) = 0
-                const float mx = mn == -INFINITY ? 0.0f : mn;
-                const float sc = expf(m[v] - mx);
+                const float sc = expf(m[v] - mn);
                 m[v] = mn;
                 s[v] *= sc;
 #pragma unroll
@@ -477,7 +476,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const bool valid = u < nv;  // a select, not a branch
-                    const float p = expf(ev[u][v] - mx);
+                    const float p = expf(ev[u][v] - mn);
                     s[v] = valid ? s[v] + p : s[v];
 #pragma unroll
                     for (int k = 0; k < VEC; ++k) {
@@ -497,8 +496,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
             for (int v = 0; v < VPL; ++v) {
                 const float mo = __shfl_xor(m[v], off), so = __shfl_xor(s[v], off);
                 const float mn = (m[v] < mo) ? mo : m[v];
-                const float mx = mn == -INFINITY ? 0.0f : mn;
-                const float c = expf(m[v] - mx), co = expf(mo - mx);
+                const float c = expf(m[v] - mn), co = expf(mo - mn);
                 s[v] = s[v] * c + so * co;
                 m[v] = mn;
 #pragma unroll
@@ -511,9 +509,7 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
 
     if (split) {
         // the chunk's (max, sum) per head, written by the lane that owns the
-        // head's first feature; (-inf, 0) where it has no other score: nothing,
-        // or NaN where no chunk of the row has (gat_reduce_kernel's exp(-inf -
-        // -inf))
+        // head's first feature
         float* prow = a.partials + static_cast<int64_t>(ch.w) * a.ldp;
 #pragma unroll
         for (int v = 0; v < VPL; ++v) {
@@ -531,8 +527,8 @@ __global__ __launch_bounds__(256) void gat_chunk_kernel(GatArgs a) {
     for (int v = 0; v < VPL; ++v) {
         if (!ok[v]) continue;
         // empty rows: s = 0 gives 0 before the bias (layers.cpp:1059); a row
-        // of -inf scores alone is NaN, its max subtracted from itself
-        const float inv = m[v] == -INFINITY && b < e ? NAN : (s[v] > 0.0f) ? 1.0f / s[v] : 0.0f;
+        // of -inf scores alone is 0 / 0, NaN as its softmax
+        const float inv = b < e ? 1.0f / s[v] : 0.0f;
         gat_store<VEC>(a, row, fo[v], acc[v], inv);
     }
 }
@@ -571,8 +567,8 @@ __global__ __launch_bounds__(256) void gat_reduce_kernel(GatArgs a) {
 #pragma unroll
             for (int k = 0; k < VEC; ++k) acc[k] = __builtin_fmaf(t[k], sc, acc[k]);
         }
-        const float inv = (S > 0.0f) ? 1.0f / S : 0.0f;
-        gat_store<VEC>(a, sp.x, fo, acc, inv);
+        // (S is 0 where every score is -inf: NaN)
+        gat_store<VEC>(a, sp.x, fo, acc, 1.0f / S);
     }
 }
 
