@@ -72,7 +72,8 @@ def test_spmm_small_plans_bitexact(gpu, restate, n, f):
 
 @pytest.mark.parametrize("f", [7, 16, 64, 100, 128])
 @pytest.mark.parametrize("n,row,long", [(9000, 3, 0), (9000, 3, 93), (9000, 3, 94),
-                                        (9000, 3, 321), (9000, 3, 322), (9000, 3, 2500), (4200, 80, 0),
+                                        (9000, 3, 321), (9000, 3, 322), (9000, 3, 2500),
+                                        (4200, 80, 0),
                                         (4200, 80, 400), (1000, 100, 0), (12400, 70, 900)])
 def test_spmm_plan_shapes_bitexact(gpu, restate, n, row, long, f):
     """Rows of one length beside one longer row, on either side of the lines

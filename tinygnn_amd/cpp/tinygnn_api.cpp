@@ -91,7 +91,7 @@ struct DevBuf {
         release();
         if (bytes == 0) bytes = 4;
         hipError_t e = hipMallocFromPoolAsync(&p, bytes, library_pool(), nullptr);
-        if (e == hipErrorOutOfMemory && tg_trim() == TG_OK) {  // what the C library keeps, given back
+        if (e == hipErrorOutOfMemory && tg_trim() == TG_OK) {  // without what the library keeps
             (void)hipGetLastError();
             e = hipMallocFromPoolAsync(&p, bytes, library_pool(), nullptr);
         }

@@ -451,7 +451,8 @@ __device__ __forceinline__ bool fast_float(const uint32_t* win, int at, int len,
     load16(win + at / 4, static_cast<uint32_t>(at) & 3, w);
     // "1.5e-03": not worth a look at its digits (lines of 2,000 such fields lost
     // a tenth of their speed to it)
-    if (len > 4 && (reinterpret_cast<const uint8_t*>(win)[at + len - 4] | 0x20) == 'e') return false;
+    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(win);
+    if (len > 4 && (bytes[at + len - 4] | 0x20) == 'e') return false;
     const uint32_t c0 = byte_of(w, 0);
     const bool lead = c0 == '-' || c0 == '+' || c0 == ' ';
     uint32_t v = 0;
